@@ -508,12 +508,13 @@ int gs_splits(const mi_moe_ctx *c, int64_t rows, int E, int64_t ncols, int glu) 
 // 42.2 / 63.9 / 86.8 / 87.9 / 88.7 -> 38.1 / 60.6 / 82.2 / 85.1 / 85.9.
 int front_split_cps(const mi_moe_ctx *c, int64_t T, int D, int E) {
     const int nch = (D + 63) / 64;
-    if (nch > 32 || T * E > FRONT_SPLIT_TE_MAX || E > 128) return 0;
+    if (T * E > FRONT_SPLIT_TE_MAX || E > 128) return 0;
     const int64_t tiles = ((T + 15) / 16) * ((E + 15) / 16);
     int nsp = 1;
     while (2 * nsp <= nch && tiles * 2 * nsp <= std::max(1, c->n_cu)) nsp *= 2;
-    if (nsp < 2 || (int64_t)nch * T * E * 2 > c->cap_z) return 0;
-    return (nch + nsp - 1) / nsp;
+    const int cps = (nch + nsp - 1) / nsp;
+    if (nsp < 2 || cps > 16 || (int64_t)nch * T * E * 2 > c->cap_z) return 0;   // (at most 16 waves a work-group)
+    return cps;
 }
 
 bool x_q8_spec(const mi_moe_ctx *c, const mi_moe_layer *L, int64_t T, Q8Out &qx) {
@@ -802,7 +803,7 @@ int run_shared(mi_moe_ctx *c, const mi_moe_layer *L, const float *x, int64_t T, 
     S.act = L->sh_act;
     const float *lg = nullptr;
     if (L->sh_gate_inp) {
-        TRY(launch_router(L->sh_gate_inp, nullptr, x, L->n_embd, T, L->n_embd, 1, c->sh_logit, st));
+        TRY(launch_front(L->sh_gate_inp, nullptr, x, L->n_embd, T, L->n_embd, 1, c->sh_logit, nullptr, st));
         lg = c->sh_logit;
     }
     TRY(launch_shared_gate(lg, T, c->sh_ids, c->sh_w, st));
@@ -1179,10 +1180,8 @@ int forward_impl(mi_moe_ctx *c, const mi_moe_layer *L, const float *x, int64_t T
             stage_end(c, "router", st);
             TRY(launch_topk_parts(parts, D, L->router_b, c->logits, T, E, K, c->sel, K, c->w, st, gt));
         } else {
-            const int rc = launch_front(L->router_w, L->router_b, xrow, D, T, D, E, c->logits, xq ? &qx : nullptr, st);
-            if (rc == -6) TRY(launch_router(L->router_w, L->router_b, xrow, D, T, D, E, c->logits, st));
-            else TRY(rc);
-            x_done = xq && rc == 0;
+            TRY(launch_front(L->router_w, L->router_b, xrow, D, T, D, E, c->logits, xq ? &qx : nullptr, st));
+            x_done = xq;
             stage_end(c, "router", st);
             TRY(launch_topk_softmax(c->logits, E, T, E, K, c->sel, K, c->w, st, gt));
         }

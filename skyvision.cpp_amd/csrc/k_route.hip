@@ -289,7 +289,10 @@ int launch_q8k_rows(const _Float16 *src, int64_t ld, int64_t nrows, int64_t K, c
 // a 16 token x 16 expert tile and whole chunks; the chunk partials meet in LDS
 // and are summed in chunk order.
 typedef double double4_t __attribute__((ext_vector_type(4)));
-constexpr int RM_MAX_CHUNKS = 32;   // D <= 2048 (64 KB of LDS partials)
+constexpr int RM_MAX_CHUNKS = 32;   // chunk partials in LDS at a time (64 KB): one group to D = 2048
+// wider rows run group after group; widths and, past one group, token counts accepted
+constexpr int RM_LIMIT_CHUNKS = 256;
+constexpr int64_t RM_LIMIT_WIDE_T = 65535;
 
 // Grid: one work-group (16 waves) per (16-token slab, 16-expert tile); the
 // slab's expert tiles run on one XCD (slab s on XCD s % 8, work-groups dealt
@@ -302,6 +305,16 @@ constexpr int RM_MAX_CHUNKS = 32;   // D <= 2048 (64 KB of LDS partials)
 // MFMA operand layout (lane (row, g): pieces 4 g .. 4 g + 3 of its row).  The
 // next chunk's loads go out once the current one is in operand registers,
 // and land while its 16 MFMAs run.
+//
+// Rows wider than 32 chunks (D > 2048) run in groups of 32: after each group
+// the work-group meets, 256 threads add its partials to their running sums in
+// chunk order, and the partials' LDS is written again (the next group's first
+// loads are in flight meanwhile).  The kernel is bound by its fp64 MFMA
+// chains and two load round trips per 16 chunks.  Measured against the form it replaces
+// for those widths (one thread per (token, expert, chunk), every lane
+// walking its own 256-byte piece of a W row): D = 2816, E = 128, T = 256, that
+// form 545 us, the layer call 963 -> 435 us; D = 2688, T = 200 412 us, 1795 ->
+// 1399 us.
 constexpr int RT_WAVES = 16;
 
 struct RtChunk {
@@ -364,7 +377,7 @@ __global__ void __launch_bounds__(1024) k_front(const float *__restrict__ W, con
     __shared__ double rparts[RM_MAX_CHUNKS * 256];   // [chunk][256]
     __shared__ float4 stage[RT_WAVES][256];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int nch = (D + 63) / 64;
+    int nch = (D + 63) / 64;
     const int net = (E + 15) / 16;
     const int lin = blockIdx.x, q = lin >> 3;
     const int64_t slab = (int64_t)(q / net) * 8 + (lin & 7);
@@ -374,17 +387,30 @@ __global__ void __launch_bounds__(1024) k_front(const float *__restrict__ W, con
     float4 *stg = stage[wave];
     RtChunk cur;
     if (wave < nch) rt_load<VEC>(cur, x, ldx, t0, T, W, e0, E, D, wave, lane);
-    for (int c = wave; c < nch; c += RT_WAVES) {
-        float xv[16], wv[16];
-        rt_transpose(cur.x, stg, lane, xv);
-        rt_transpose(cur.w, stg, lane, wv);
-        if (c + RT_WAVES < nch) rt_load<VEC>(cur, x, ldx, t0, T, W, e0, E, D, c + RT_WAVES, lane);
-        double4_t part = {0.0, 0.0, 0.0, 0.0};
+    double acc = 0.0;   // threads 0-255: the running sum of the groups before the last
+    for (int g0 = 0;;) {
+        const int g1 = g0 + RM_MAX_CHUNKS < nch ? g0 + RM_MAX_CHUNKS : nch;
+        for (int c = g0 + wave; c < g1; c += RT_WAVES) {
+            float xv[16], wv[16];
+            rt_transpose(cur.x, stg, lane, xv);
+            rt_transpose(cur.w, stg, lane, wv);
+            if (c + RT_WAVES < nch) rt_load<VEC>(cur, x, ldx, t0, T, W, e0, E, D, c + RT_WAVES, lane);
+            double4_t part = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-        for (int s2 = 0; s2 < 16; ++s2)
-            part = __builtin_amdgcn_mfma_f64_16x16x4f64((double)xv[s2], (double)wv[s2], part, 0, 0, 0);
+            for (int s2 = 0; s2 < 16; ++s2)
+                part = __builtin_amdgcn_mfma_f64_16x16x4f64((double)xv[s2], (double)wv[s2], part, 0, 0, 0);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) rparts[c * 256 + lane * 4 + r] = part[r];
+            for (int r = 0; r < 4; ++r) rparts[(c - g0) * 256 + lane * 4 + r] = part[r];
+        }
+        if (g1 == nch) {
+            nch -= g0;   // the last group's chunks, added below
+            break;
+        }
+        __syncthreads();
+        if (threadIdx.x < 256)
+            for (int c = 0; c < RM_MAX_CHUNKS; ++c) acc = acc + rparts[c * 256 + threadIdx.x];
+        __syncthreads();   // the partials are rewritten next
+        g0 = g1;
     }
     if (o.q8 || o.xh) {
         const int nb = D / QK, ngrp = (nb + 3) >> 2;
@@ -404,7 +430,6 @@ __global__ void __launch_bounds__(1024) k_front(const float *__restrict__ W, con
         const int64_t tt = t0 + 4 * r + (l >> 4);
         const int ee = e0 + (l & 15);
         // chunk partials added in chunk order, eight loads in flight
-        double acc = 0.0;
         int c = 0;
         for (; c + 8 <= nch; c += 8) {
             double v[8];
@@ -476,42 +501,11 @@ __global__ void __launch_bounds__(1024) k_front_parts(const float *__restrict__ 
     }
 }
 
-// generic form (any D): thread (expert, chunk) computes one partial
-__global__ void __launch_bounds__(256) k_router_split(const float *__restrict__ W, const float *__restrict__ bias,
-                                                      const float *__restrict__ x, int64_t ldx, int D, int E,
-                                                      int nch, int epb, float *__restrict__ logits) {
-    __shared__ double parts[256];
-    const int tid = threadIdx.x;
-    const int el = tid / nch, c = tid % nch;
-    const int64_t t = blockIdx.y;
-    const int e = blockIdx.x * epb + el;
-    const bool act = el < epb && e < E;
-    double part = 0.0;
-    if (act) {
-        const float *w = W + (int64_t)e * D;
-        const float *xt = x + t * ldx;
-        for (int s = 0; s < 16; ++s)
-            for (int g = 0; g < 4; ++g) {
-                const int dd = 64 * c + 16 * g + s;
-                if (dd < D) part = fma((double)w[dd], (double)xt[dd], part);
-            }
-    }
-    parts[tid] = part;
-    __syncthreads();
-    if (act && c == 0) {
-        double acc = 0.0;
-        for (int j = 0; j < nch; j++) acc = acc + parts[el * nch + j];
-        float v = (float)acc;
-        if (bias) v = v + bias[e];
-        logits[t * E + e] = v;
-    }
-}
-
 int launch_front(const float *W, const float *b, const float *x, int64_t ldx, int64_t T, int D, int E,
                  float *logits, const Q8Out *qx, hipStream_t st) {
     if (T <= 0) return 0;
     const int nch = (D + 63) / 64;
-    if (nch > RM_MAX_CHUNKS || T > (int64_t)1 << 30) return -6;
+    if (nch > RM_LIMIT_CHUNKS || T > (nch > RM_MAX_CHUNKS ? RM_LIMIT_WIDE_T : (int64_t)1 << 30)) return -6;
     if (qx && D % QK) return -6;
     const bool vec = (D % 64 == 0) && (ldx % 4 == 0) && ((uintptr_t)x % 16 == 0) && ((uintptr_t)W % 16 == 0);
     const int64_t net = (E + 15) / 16, nslab = (T + 15) / 16;
@@ -534,7 +528,7 @@ int launch_front_parts(const float *W, const float *x, int64_t ldx, int64_t T, i
                        double *parts, const Q8Out *qx, hipStream_t st) {
     if (T <= 0) return 0;
     const int nch = (D + 63) / 64;
-    if (nch > RM_MAX_CHUNKS || cps < 1 || cps > RT_WAVES || T > (int64_t)1 << 24) return -6;
+    if (nch > RM_LIMIT_CHUNKS || cps < 1 || cps > RT_WAVES || T > (int64_t)1 << 24) return -6;
     if (qx && D % QK) return -6;
     const bool vec = (D % 64 == 0) && (ldx % 4 == 0) && ((uintptr_t)x % 16 == 0) && ((uintptr_t)W % 16 == 0);
     const int64_t nsp = (nch + cps - 1) / cps, net = (E + 15) / 16, nslab = (T + 15) / 16;
@@ -548,19 +542,6 @@ int launch_front_parts(const float *W, const float *x, int64_t ldx, int64_t T, i
         hipLaunchKernelGGL((k_front_parts<true, XO_ANY>), grid, block, 0, st, W, x, ldx, T, D, E, cps, parts, o);
     else
         hipLaunchKernelGGL((k_front_parts<false, XO_ANY>), grid, block, 0, st, W, x, ldx, T, D, E, cps, parts, o);
-    return hip_check_launch();
-}
-
-int launch_router(const float *W, const float *b, const float *x, int64_t ldx, int64_t T, int D, int E,
-                  float *logits, hipStream_t st) {
-    if (T <= 0) return 0;
-    const int nch = (D + 63) / 64;
-    if (nch <= RM_MAX_CHUNKS && T <= (int64_t)1 << 30)
-        return launch_front(W, b, x, ldx, T, D, E, logits, nullptr, st);
-    if (nch > 256 || T > 65535) return -6;
-    const int epb = 256 / nch;
-    hipLaunchKernelGGL(k_router_split, dim3((unsigned)((E + epb - 1) / epb), (unsigned)T), dim3(256), 0, st, W, b,
-                       x, ldx, D, E, nch, epb, logits);
     return hip_check_launch();
 }
 
@@ -607,15 +588,25 @@ __global__ void __launch_bounds__(64) k_topk_parts(const double *__restrict__ pa
     const int lane = threadIdx.x;
     const int64_t t = blockIdx.x;
     const int64_t cs = T * E;
-    double pv[NPER][RM_MAX_CHUNKS];
+    double acc[NPER];
 #pragma unroll
-    for (int i = 0; i < NPER; ++i) {
-        const int e = lane + 64 * i;
-        const double *p = parts + t * E + (e < E ? e : 0);
-        // branch-free: chunks past nch re-load the last one (never added), so
-        // no load waits for an earlier one (nch >= 1)
+    for (int i = 0; i < NPER; ++i) acc[i] = 0.0;
+    for (int g0 = 0; g0 < nch; g0 += RM_MAX_CHUNKS) {
+        double pv[NPER][RM_MAX_CHUNKS];
 #pragma unroll
-        for (int c = 0; c < RM_MAX_CHUNKS; ++c) pv[i][c] = p[(int64_t)(c < nch ? c : nch - 1) * cs];
+        for (int i = 0; i < NPER; ++i) {
+            const int e = lane + 64 * i;
+            const double *p = parts + t * E + (e < E ? e : 0);
+            // branch-free: chunks past nch re-load the last one (never added), so
+            // no load waits for an earlier one (nch >= 1)
+#pragma unroll
+            for (int c = 0; c < RM_MAX_CHUNKS; ++c) pv[i][c] = p[(int64_t)(g0 + c < nch ? g0 + c : nch - 1) * cs];
+        }
+#pragma unroll
+        for (int i = 0; i < NPER; ++i)
+#pragma unroll
+            for (int c = 0; c < RM_MAX_CHUNKS; ++c)
+                if (g0 + c < nch) acc[i] = acc[i] + pv[i][c];
     }
     float raw[TOPK_MAX_PER_LANE];
 #pragma unroll
@@ -623,11 +614,7 @@ __global__ void __launch_bounds__(64) k_topk_parts(const double *__restrict__ pa
 #pragma unroll
     for (int i = 0; i < NPER; ++i) {
         const int e = lane + 64 * i;
-        double acc = 0.0;
-#pragma unroll
-        for (int c = 0; c < RM_MAX_CHUNKS; ++c)
-            if (c < nch) acc = acc + pv[i][c];
-        float v = (float)acc;
+        float v = (float)acc[i];
         if (e < E) {
             if (bias) v = v + bias[e];
             raw[i] = v;
@@ -649,7 +636,7 @@ int launch_topk_parts(const double *parts, int D, const float *bias, float *logi
     if (E > 128 || K > 64 || K > E || K <= 0 || T > 0x7fffffff) return -6;
     if (gt.kind < 0 || gt.kind > 2) return -6;
     const int nch = (D + 63) / 64;
-    if (nch > RM_MAX_CHUNKS) return -6;
+    if (nch > RM_LIMIT_CHUNKS) return -6;
     if (E <= 64)
         hipLaunchKernelGGL(k_topk_parts<1>, dim3((unsigned)T), dim3(64), 0, st, parts, nch, bias, logits, T, E, K, sel,
                            ld_sel, w, gt);

@@ -529,10 +529,30 @@ bool x_q8_spec(const mi_moe_ctx *c, const mi_moe_layer *L, int64_t T, Q8Out &qx)
     return true;
 }
 
-// routed FFN body of a layer with Q4_0 / Q5_0 / Q8_0 / F16 tables (k_b32.hip):
-// the rows converted to each product's ggml vec_dot_type (Q8_0 or fp16), the
-// grouped GEMV below the GEMM threshold, the grouped MFMA GEMM above it, GLU
-// rows in fp32, fp32 slot rows into the combine.  Arguments as run_experts.
+int64_t round_up(int64_t n, int64_t to) { return (n + to - 1) / to * to; }
+
+// Row tiles of the grouped GEMM of the 32-value types and F16 (k_gb.hip): 128
+// rows above 16 dispatched rows per expert, else 32.  Layer us, Q8_0, same
+// box, 32 / 64 / 128-row tiles: qwen3omni T = 100 (6 rows per expert) 206 /
+// 222 / 207, T = 300 (19) 252 / 241 / 222, T = 600 (38) 332 / 275 / 253;
+// moondream3 T = 160 (20) 188 / 175 / 161.  A call of few work-groups (a
+// shared expert) keeps the small tiles, which are four times as many.
+int gb_bm(const mi_moe_ctx *c, int64_t rows, int E, int64_t ncols) {
+    const int64_t wgs = (rows / GB_BM_LARGE + E) * (ncols / 256);
+    return rows > 16 * (int64_t)E && wgs >= c->n_cu ? GB_BM_LARGE : GB_BM_SMALL;
+}
+// the grouped GEMM reads its activation rows through 32-bit buffer offsets:
+// tokens per pass of a call whose rows hold at most `halfs` fp16 values per
+// token (larger calls run in passes)
+int64_t gb_max_tokens(int64_t halfs) { return GB_MAX_X / (2 * halfs); }
+bool gb_strides_ok(const mi_tensor &t) { return (int64_t)t.nb[1] <= GB_MAX_ROW_BYTES; }
+
+// routed FFN body of a layer with Q4_0 / Q5_0 / Q8_0 / F16 tables: the rows
+// converted to each product's ggml vec_dot_type (Q8_0 or fp16), fp32 slot
+// rows into the combine.  Below the GEMM threshold the grouped GEMV
+// (k_b32.hip), GLU rows in fp32; above it the grouped MFMA GEMM (k_gb.hip),
+// whose gate/up launch writes the down product's operand rows itself.
+// Arguments as run_experts.
 int run_experts_b32(mi_moe_ctx *c, const mi_moe_layer *L, const float *x, int64_t T, const int32_t *ids_gu,
                     const int32_t *ids_dn, const float *w, const float *res, float *out, hipStream_t st,
                     bool check_ids, const float *add) {
@@ -541,48 +561,83 @@ int run_experts_b32(mi_moe_ctx *c, const mi_moe_layer *L, const float *x, int64_
     const int max_active = (int)std::min<int64_t>(E, rows);
     const bool same_ids = ids_gu == ids_dn;
     const bool gated = act_gated(L->act);
-    const bool gemm = use_gemm_wide(c, T, K, E);
-    const int max_tiles = (int)((rows + G4_BM - 1) / G4_BM + max_active);
-    TRY(launch_dispatch(ids_gu, T, K, E, G4_BM, 1, c->disp[0].view(), st));
-    if (!same_ids) TRY(launch_dispatch(ids_dn, T, K, E, G4_BM, 1, c->disp[1].view(), st));
+    // (row strides past the GEMM's 32-bit offsets keep the GEMV)
+    const bool gemm = use_gemm_wide(c, T, K, E) && gb_strides_ok(L->gate) && gb_strides_ok(L->down) &&
+                      (!gated || L->fused_gate_up || gb_strides_ok(L->up));
+    const int64_t ldx = round_up(D, 64), ldi = round_up(I, 64);
+    const int64_t tmax = gb_max_tokens(std::max(ldx, K * ldi));
+    if (gemm && T > tmax) {
+        // in passes; then the dispatch of the whole call, whose counts, offsets and lists the caller may read
+        for (int64_t t0 = 0; t0 < T; t0 += tmax) {
+            const int64_t n = std::min(tmax, T - t0);
+            TRY(run_experts_b32(c, L, x + t0 * D, n, ids_gu + t0 * K, ids_dn + t0 * K, w + t0 * K,
+                                res ? res + t0 * D : nullptr, out + t0 * D, st, check_ids, add ? add + t0 * D : nullptr));
+        }
+        DispBuf whole = c->disp[0];
+        whole.bad_total = nullptr;   // (counted by the passes)
+        return launch_dispatch(ids_gu, T, K, E, gb_bm(c, rows, E, D), 1, whole.view(), st);
+    }
+    const int bm = gemm ? gb_bm(c, rows, E, D) : G4_BM;
+    const int max_tiles = (int)((rows + bm - 1) / bm + max_active);
+    TRY(launch_dispatch(ids_gu, T, K, E, bm, 1, c->disp[0].view(), st));
+    if (!same_ids) TRY(launch_dispatch(ids_dn, T, K, E, bm, 1, c->disp[1].view(), st));
     const DispBuf &dg = c->disp[0];
     const DispBuf &dd = same_ids ? c->disp[0] : c->disp[1];
     stage_end(c, "dispatch", st);
     // an activation set in the operand form of a consumer type on this path
-    auto prep_for = [&](int wtype, ActBuf &ab, int pre_act) {
+    auto prep_for = [&](int wtype, ActBuf &ab, int64_t width, int pre_act) {
         B32Prep o;
         o.pre_act = pre_act;
+        o.ldo = gemm ? round_up(width, 64) : width;
         if (wtype == MI_TYPE_F16) { o.mode = B32_PREP_F16; o.xh = ab.h; }
         else if (gemm) { o.mode = B32_PREP_DQ; o.xh = ab.h; }
         else { o.mode = B32_PREP_CODES; o.q8 = ab.q8; o.dh = (uint16_t *)ab.bs; }
         return o;
     };
-    auto args_for = [&](const ExpertMat &a, const DispBuf &d, const ActBuf &ab, int ne11) {
-        B32Args g = {};
-        g.a = a; g.ne11 = ne11; g.K = K; g.act = L->act; g.I = I;
-        g.q8 = ab.q8; g.dh = (const uint16_t *)ab.bs; g.xh = ab.h;
-        g.counts = d.counts; g.offsets = d.offsets; g.perm = d.perm; g.active_e = d.active_e;
-        g.n_active = d.n_active; g.max_active = max_active;
-        g.tile_e = d.tile_e; g.tile_start = d.tile_start; g.tile_rows = d.tile_rows; g.n_tiles = d.n_tiles;
-        g.max_tiles = max_tiles;
-        return g;
-    };
-    TRY(launch_prep_b32(x, D, T, D, prep_for(L->gate.type, c->ax, 0), st));
+    TRY(launch_prep_b32(x, D, T, D, prep_for(L->gate.type, c->ax, D, 0), st));
     stage_end(c, "q8_x", st);
-    B32Args a = args_for(as_mat(L->gate), dg, c->ax, 1);
-    if (gated && !L->fused_gate_up) a.b = as_mat(L->up);
-    a.glu = gated ? 1 : 0;
-    a.fused = L->fused_gate_up;
-    a.y = c->f1; a.ldy = I; a.ncols = I;
-    TRY(gemm ? launch_gemm_b32(a, st) : launch_gemv_b32(a, st));
-    stage_end(c, "gate_up", st);
-    // one product (relu^2 experts): its rows are squared on the way to the down operand
-    TRY(launch_prep_b32(c->f1, I, rows, I, prep_for(L->down.type, c->aact, gated ? 0 : MI_ACT_RELU_SQR), st));
-    stage_end(c, "q8_act", st);
-    B32Args d = args_for(as_mat(L->down), dd, c->aact, K);
-    d.glu = 0;
-    d.y = c->z; d.ldy = D; d.ncols = D;
-    TRY(gemm ? launch_gemm_b32(d, st) : launch_gemv_b32(d, st));
+    if (gemm) {
+        GBArgs a = {};
+        a.a = as_mat(L->gate);
+        if (gated && !L->fused_gate_up) a.b = as_mat(L->up);
+        a.glu = gated ? 1 : 0; a.relu_sqr = gated ? 0 : 1; a.fused = L->fused_gate_up; a.act = L->act; a.I = I;
+        a.xh = c->ax.h; a.ldx = ldx; a.xrows = T; a.ne11 = 1; a.K = K;
+        a.perm = dg.perm; a.tile_e = dg.tile_e; a.tile_start = dg.tile_start; a.tile_rows = dg.tile_rows;
+        a.n_tiles = dg.n_tiles; a.max_tiles = max_tiles; a.bm = bm;
+        a.ncols = I; a.xo = c->aact.h; a.ldo = ldi; a.next_f16 = L->down.type == MI_TYPE_F16;
+        TRY(launch_gb(a, st));
+        stage_end(c, "gate_up", st);
+        GBArgs d = {};
+        d.a = as_mat(L->down);
+        d.xh = c->aact.h; d.ldx = ldi; d.xrows = rows; d.ne11 = K; d.K = K;
+        d.perm = dd.perm; d.tile_e = dd.tile_e; d.tile_start = dd.tile_start; d.tile_rows = dd.tile_rows;
+        d.n_tiles = dd.n_tiles; d.max_tiles = max_tiles; d.bm = bm;
+        d.y = c->z; d.ldy = D; d.ncols = D;
+        TRY(launch_gb(d, st));
+    } else {
+        auto args_for = [&](const ExpertMat &a, const DispBuf &d, const ActBuf &ab, int ne11) {
+            B32Args g = {};
+            g.a = a; g.ne11 = ne11; g.K = K; g.act = L->act; g.I = I;
+            g.q8 = ab.q8; g.dh = (const uint16_t *)ab.bs; g.xh = ab.h;
+            g.counts = d.counts; g.offsets = d.offsets; g.perm = d.perm; g.active_e = d.active_e;
+            g.n_active = d.n_active; g.max_active = max_active;
+            return g;
+        };
+        B32Args a = args_for(as_mat(L->gate), dg, c->ax, 1);
+        if (gated && !L->fused_gate_up) a.b = as_mat(L->up);
+        a.glu = gated ? 1 : 0;
+        a.fused = L->fused_gate_up;
+        a.y = c->f1; a.ldy = I; a.ncols = I;
+        TRY(launch_gemv_b32(a, st));
+        stage_end(c, "gate_up", st);
+        // one product (relu^2 experts): its rows are squared on the way to the down operand
+        TRY(launch_prep_b32(c->f1, I, rows, I, prep_for(L->down.type, c->aact, I, gated ? 0 : MI_ACT_RELU_SQR), st));
+        stage_end(c, "q8_act", st);
+        B32Args d = args_for(as_mat(L->down), dd, c->aact, K);
+        d.glu = 0;
+        d.y = c->z; d.ldy = D; d.ncols = D;
+        TRY(launch_gemv_b32(d, st));
+    }
     stage_end(c, "down", st);
     CombineIds ci;
     if (check_ids) { ci.a = ids_gu; ci.b = ids_dn; ci.E = E; }
@@ -1376,33 +1431,54 @@ int mi_mul_mat_id(mi_moe_ctx *c, const mi_tensor *as, const mi_tensor *b, const 
     HIP_TRY(hipSetDevice(c->device));
     hipStream_t st = (hipStream_t)stream;
     const int64_t rows = T * n_used;
+    // the grouped GEMM of the 32-value types and F16, in passes past its 32-bit offsets
+    const bool gb = is_b32f(as->type) && use_gemm_wide(c, T, (int)n_used, (int)E) && gb_strides_ok(*as);
+    const int64_t ldx = round_up(Kin, 64), tmax = gb_max_tokens(ne11 * ldx);
+    if (gb && T > tmax) {
+        for (int64_t t0 = 0; t0 < T; t0 += tmax) {
+            const int64_t n = std::min(tmax, T - t0);
+            mi_tensor bt = *b, it = *ids, dt = *dst;
+            bt.data = (float *)b->data + t0 * ne11 * Kin; bt.ne[2] = n;
+            it.data = (int32_t *)ids->data + t0 * n_used; it.ne[1] = n;
+            dt.data = (float *)dst->data + t0 * n_used * N; dt.ne[2] = n;
+            TRY(mi_mul_mat_id(c, as, &bt, &it, &dt, stream));
+        }
+        return MI_MOE_OK;
+    }
     const int max_active = (int)std::min<int64_t>(E, rows);
-    const int max_tiles = (int)((rows + G4_BM - 1) / G4_BM + max_active);
+    const int bm = gb ? gb_bm(c, rows, (int)E, N) : G4_BM;
+    const int max_tiles = (int)((rows + bm - 1) / bm + max_active);
     const DispBuf &dsp = c->disp[0];
     Dispatch dv = dsp.view();
     dv.zero_rows = (float *)dst->data;   // the rows of ids outside [0, E): zeros
     dv.zero_ld = N;
     dv.zero_n = N;
-    TRY(launch_dispatch((const int32_t *)ids->data, T, (int)n_used, (int)E, G4_BM, 1, dv, st));
+    TRY(launch_dispatch((const int32_t *)ids->data, T, (int)n_used, (int)E, bm, 1, dv, st));
     const ExpertMat M = as_mat(*as);
     const float *bp = (const float *)b->data;
     if (is_b32f(as->type)) {
         // b in the table type's vec_dot_type (Q8_0 or fp16), then the grouped GEMV or GEMM
-        const bool gemm = use_gemm_wide(c, T, (int)n_used, (int)E);
         B32Prep o;
+        o.ldo = gb ? ldx : Kin;
         if (as->type == MI_TYPE_F16) { o.mode = B32_PREP_F16; o.xh = c->ax.h; }
-        else if (gemm) { o.mode = B32_PREP_DQ; o.xh = c->ax.h; }
+        else if (gb) { o.mode = B32_PREP_DQ; o.xh = c->ax.h; }
         else { o.mode = B32_PREP_CODES; o.q8 = c->ax.q8; o.dh = (uint16_t *)c->ax.bs; }
         TRY(launch_prep_b32(bp, Kin, T * ne11, Kin, o, st));
+        if (gb) {
+            GBArgs a = {};
+            a.a = M; a.xh = c->ax.h; a.ldx = ldx; a.xrows = T * ne11; a.ne11 = (int)ne11; a.K = (int)n_used;
+            a.perm = dsp.perm; a.tile_e = dsp.tile_e; a.tile_start = dsp.tile_start; a.tile_rows = dsp.tile_rows;
+            a.n_tiles = dsp.n_tiles; a.max_tiles = max_tiles; a.bm = bm;
+            a.y = (float *)dst->data; a.ldy = N; a.ncols = N;
+            return launch_gb(a, st);
+        }
         B32Args a = {};
         a.a = M; a.glu = 0; a.ne11 = (int)ne11; a.K = (int)n_used;
         a.q8 = c->ax.q8; a.dh = (const uint16_t *)c->ax.bs; a.xh = c->ax.h;
         a.counts = dsp.counts; a.offsets = dsp.offsets; a.perm = dsp.perm; a.active_e = dsp.active_e;
         a.n_active = dsp.n_active; a.max_active = max_active;
-        a.tile_e = dsp.tile_e; a.tile_start = dsp.tile_start; a.tile_rows = dsp.tile_rows; a.n_tiles = dsp.n_tiles;
-        a.max_tiles = max_tiles;
         a.y = (float *)dst->data; a.ldy = N; a.ncols = N;
-        return gemm ? launch_gemm_b32(a, st) : launch_gemv_b32(a, st);
+        return launch_gemv_b32(a, st);
     }
     if (as->type == MI_TYPE_F32) {
         GemvArgs a = {};

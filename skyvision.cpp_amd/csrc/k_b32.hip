@@ -15,14 +15,8 @@
 //    rows (GEMM, and F16's GEMV),
 //  * the grouped GEMV (decode): 8 lanes per weight row, each lane one 32-value
 //    block per 256 values, integer dots on v_dot4_i32_i8 / fp16 pairs on
-//    v_dot2_f32_f16,
-//  * the grouped GEMM (prefill) on v_mfma_f32_32x32x16_f16: a work-group owns
-//    a balanced tile of up to 192 dispatched rows of one expert and 128 weight
-//    rows (GLU: 64 gate and the 64 matching up rows), each wave 32 of them
-//    against all the tile's rows (6 MFMA tiles, one dequantized weight operand
-//    feeds all of them); activations staged through LDS 64 K values at a
-//    time (double buffered, 16-byte chunks swizzled by row), weights loaded
-//    into registers one stage ahead and dequantized to fp16 in registers.
+//    v_dot2_f32_f16.
+// The grouped GEMM (prefill) is k_gb.hip.
 //
 // Block layouts (ggml block_q4_0 / q5_0 / q8_0, no padding, so blocks start
 // at any even byte):
@@ -30,12 +24,11 @@
 //   Q5_0 22 B: d f16 | qh u32 | qs[16]   5th bit of value j: bit j of qh;                 x = d (q - 16)
 //   Q8_0 34 B: d f16 | qs[32] i8                                                          x = d q
 #include "act.hpp"
+#include "b32.hpp"
 #include "common.hpp"
 #include "launch.hpp"
 
 namespace mimoe {
-
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 template <int WT> struct B32Fmt;
 template <> struct B32Fmt<2> { static constexpr int BYTES = 18, WORDS = 5, OFF = 8; };    // Q4_0
@@ -165,47 +158,62 @@ int launch_quantize_b32(int type, const float *src, void *dst, int64_t nblocks, 
 // ------------------------------------------------------------------ activations
 // Rows of K values (K % 32 == 0, row r at src + r * ld) into the operand form
 // of a consumer weight type (B32Prep): Q8_0 codes [r][K] and fp16 scales
-// [r][K/32] (GEMV of Q4_0 / Q5_0 / Q8_0), fp16(d q) rows [r][K] (their GEMM),
-// or fp16(x) rows [r][K] (F16, both paths).  One block per 32 lanes; the Q8_0
-// scale and codes are the oracle's bit for bit.
-template <typename S>
-__global__ void __launch_bounds__(256) k_prep_b32(const S *src, int64_t ld, int64_t nrows, int64_t K, B32Prep o) {
-    const int64_t nbr = K / 32;
-    const int64_t blk = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 5;
-    const int j = threadIdx.x & 31;
-    if (blk >= nrows * nbr) return;   // a whole half-wave leaves together
-    const int64_t r = blk / nbr, b = blk - r * nbr;
-    float v = (float)src[r * ld + 32 * b + j];
-    if (o.pre_act == 4) {   // ggml_sqr(ggml_relu(u)) before the quantization
-        const float t = v > 0.f ? v : 0.f;
-        v = t * t;
-    }
-    const int64_t at = r * K + 32 * b + j;
-    if (o.mode == B32_PREP_F16) {
-        o.xh[at] = __builtin_bit_cast(_Float16, (uint16_t)f32_to_fp16_bits(v));
-        return;
-    }
-    float amax = fabsf(v);
+// [r][K/32] (GEMV of Q4_0 / Q5_0 / Q8_0), fp16(d q) rows [r][ldo] (their GEMM),
+// or fp16(x) rows [r][ldo] (F16, both paths); the Q8_0 scale and codes are the
+// oracle's bit for bit.  Memory-bound; 8 values per thread, four threads per
+// block (16-byte loads and stores; 600 rows of 2048: 5.0 us,
+// one value per lane 8.5).
+// VEC: 16-byte aligned rows.
+template <bool VEC>
+__global__ void __launch_bounds__(256) k_prep_b32(const float *src, int64_t ld, int64_t nrows, int64_t K, B32Prep o) {
+    const int64_t w = o.mode == B32_PREP_CODES ? K : o.ldo, nch = w / 8;   // 8-value chunks per row (a multiple of 4)
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= nrows * nch) return;   // the four threads of a block leave together
+    const int64_t r = i / nch, c = i - r * nch;
+    float v[8];
+    if (8 * c < K) {
+        const float *x = src + r * ld + 8 * c;
+        if constexpr (VEC) {
+            const float4 a = *(const float4 *)x, b = *(const float4 *)(x + 4);
+            v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+        } else {
 #pragma unroll
-    for (int s = 1; s < 32; s <<= 1) amax = fmaxf(amax, __shfl_xor(amax, s, 32));
-    const float d = amax / 127.0f;
-    const float id = d != 0.0f ? 1.0f / d : 0.0f;
-    const int q = (int)roundf(v * id);
-    const uint32_t dh = f32_to_fp16_bits(d);
-    if (o.mode == B32_PREP_CODES) {
-        o.q8[at] = (int8_t)q;
-        if (j == 0) o.dh[r * nbr + b] = (uint16_t)dh;
+            for (int j = 0; j < 8; ++j) v[j] = x[j];
+        }
     } else {
-        o.xh[at] = (_Float16)(fp16_bits_to_f32(dh) * (float)q);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = 0.f;
+    }
+    if (o.pre_act == 4) {   // ggml_sqr(ggml_relu(u)) before the quantization
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = relu_sqr(v[j]);
+    }
+    if (o.mode == B32_PREP_CODES) {
+        int q[8];
+        uint32_t dh;
+        b32_q8_codes(v, q, dh);
+        uint32_t lo = 0, hi = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            lo |= (uint32_t)(q[j] & 0xff) << (8 * j);
+            hi |= (uint32_t)(q[4 + j] & 0xff) << (8 * j);
+        }
+        *(uint2 *)(o.q8 + r * K + 8 * c) = make_uint2(lo, hi);
+        if ((c & 3) == 0) o.dh[r * (K / 32) + c / 4] = (uint16_t)dh;
+    } else {
+        *(uint4 *)(o.xh + r * o.ldo + 8 * c) = o.mode == B32_PREP_F16 ? b32_f16x8(v) : b32_q8x8(v);
     }
 }
 
 int launch_prep_b32(const float *src, int64_t ld, int64_t nrows, int64_t K, const B32Prep &o, hipStream_t st) {
     if (nrows <= 0) return 0;
     if (K % 32) return -6;
-    const int64_t threads = nrows * K;
-    hipLaunchKernelGGL(k_prep_b32<float>, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st, src, ld, nrows,
-                       K, o);
+    if (o.mode != B32_PREP_CODES && (o.ldo < K || o.ldo % 32)) return -6;
+    const int64_t threads = nrows * ((o.mode == B32_PREP_CODES ? K : o.ldo) / 8);
+    const dim3 grid((unsigned)((threads + 255) / 256));
+    const bool vec = ld % 4 == 0 && (uintptr_t)src % 16 == 0;
+    if (vec) hipLaunchKernelGGL(k_prep_b32<true>, grid, dim3(256), 0, st, src, ld, nrows, K, o);
+    else hipLaunchKernelGGL(k_prep_b32<false>, grid, dim3(256), 0, st, src, ld, nrows, K, o);
     return hip_check_launch();
 }
 
@@ -297,214 +305,7 @@ __global__ void __launch_bounds__(256) k_gemv_b32(B32Args g) {
     }
 }
 
-// ------------------------------------------------------------------ GEMM
-constexpr int GB_BM = G4_BM;        // rows per tile (balanced dispatch tiles)
-constexpr int GB_RT = GB_BM / 32;   // row tiles of 32
-constexpr int GB_BK = 64;           // K values per stage
-constexpr int GB_ACH = GB_BM * (GB_BK / 8) / 256;   // 16-byte activation chunks per thread per stage
-
-// this lane's weight operands of one stage: for K16 step s, K values
-// k0 + 16 s + 8 h + (0..7) of its row (h = lane / 32), as fp16
-template <int WT> struct GBRaw { uint32_t w0[B32Fmt<WT>::WORDS], w1[B32Fmt<WT>::WORDS]; uint32_t mis0, mis1; };
-template <> struct GBRaw<1> { uint4 v[4]; };
-
-template <int WT>
-__device__ inline void gb_load(const uint8_t *row, int64_t k0, int64_t Kin, int h, GBRaw<WT> &r) {
-    if constexpr (WT == 1) {
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            const int64_t k = k0 + 16 * s + 8 * h;
-            r.v[s] = k < Kin ? *(const uint4 *)(row + 2 * k) : make_uint4(0, 0, 0, 0);
-        }
-    } else {
-        const int64_t blk = k0 / 32;
-        b32_words<WT>(row + (int64_t)B32Fmt<WT>::BYTES * blk, r.w0, r.mis0);
-        if (blk + 1 < Kin / 32) {
-            b32_words<WT>(row + (int64_t)B32Fmt<WT>::BYTES * (blk + 1), r.w1, r.mis1);
-        } else {
-#pragma unroll
-            for (int i = 0; i < B32Fmt<WT>::WORDS; ++i) r.w1[i] = 0u;   // d = 0: zero weights
-            r.mis1 = 0u;
-        }
-    }
-}
-
-// 4 unsigned byte codes (+ bias making them unsigned) -> 2 half2 of (q - off) * d
-__device__ inline void gb_bytes_h(uint32_t x, float off, half2_t d2, half2_t &lo, half2_t &hi) {
-    // bytes b0..b3 into fp16 1024 + b (exact), then - (1024 + off), then * d
-    const uint32_t p01 = __builtin_amdgcn_perm(0x64646464u, x, 0x04010400u);
-    const uint32_t p23 = __builtin_amdgcn_perm(0x64646464u, x, 0x04030402u);
-    const _Float16 c = (_Float16)(1024.0f + off);
-    const half2_t cc = {c, c};
-    lo = (__builtin_bit_cast(half2_t, p01) - cc) * d2;
-    hi = (__builtin_bit_cast(half2_t, p23) - cc) * d2;
-}
-
-template <int WT, int S>
-__device__ inline half8_t gb_operand(const GBRaw<WT> &r, int h) {
-    if constexpr (WT == 1) {
-        return __builtin_bit_cast(half8_t, r.v[S]);
-    } else {
-        const auto &w = S < 2 ? r.w0 : r.w1;
-        const uint32_t mis = S < 2 ? r.mis0 : r.mis1;
-        const _Float16 dh = (_Float16)b32_d(w[0], mis);
-        const half2_t d2 = {dh, dh};
-        // values v0 .. v0 + 7 of the block, v0 = 16 (S & 1) + 8 h: groups of 4
-        // i0 = 4 (S & 1) + 2 h and i0 + 1
-        constexpr int J = 4 * (S & 1);
-        uint32_t c0 = h ? b32_codes4<WT, J + 2>(w, mis) : b32_codes4<WT, J>(w, mis);
-        uint32_t c1 = h ? b32_codes4<WT, J + 3>(w, mis) : b32_codes4<WT, J + 1>(w, mis);
-        float off;
-        if constexpr (WT == 8) {
-            c0 ^= 0x80808080u;   // signed -> q + 128
-            c1 ^= 0x80808080u;
-            off = 128.0f;
-        } else {
-            off = WT == 2 ? 8.0f : 16.0f;
-        }
-        half2_t a0, a1, a2, a3;
-        gb_bytes_h(c0, off, d2, a0, a1);
-        gb_bytes_h(c1, off, d2, a2, a3);
-        const u32x4 o = {__builtin_bit_cast(uint32_t, a0), __builtin_bit_cast(uint32_t, a1),
-                         __builtin_bit_cast(uint32_t, a2), __builtin_bit_cast(uint32_t, a3)};
-        return __builtin_bit_cast(half8_t, o);
-    }
-}
-
-template <int WT, bool GLU>
-__global__ void __launch_bounds__(256) k_gemm_b32(B32Args g) {
-    __shared__ __attribute__((aligned(16))) _Float16 As[2][GB_BM * GB_BK];   // 2 x 24 KB
-    __shared__ int s_row[GB_BM];   // activation row of each tile row
-    __shared__ int s_p[GB_BM];     // output row (slot index) of each tile row, -1 past the tile
-    const int tile = blockIdx.y;
-    if (tile >= *g.n_tiles) return;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
-    const int e = g.tile_e[tile], start = g.tile_start[tile], mrows = g.tile_rows[tile];
-    const int nrt = (mrows + 31) >> 5;
-    // this lane's weight row and output column
-    int64_t col;
-    const ExpertMat *M = &g.a;
-    int64_t wrow;
-    if (GLU) {
-        col = (int64_t)blockIdx.x * 64 + 32 * (wave & 1) + l32;
-        wrow = col;
-        if (wave >= 2) {
-            if (g.fused) wrow = g.I + col;
-            else M = &g.b;
-        }
-    } else {
-        col = (int64_t)blockIdx.x * 128 + 32 * wave + l32;
-        wrow = col;
-    }
-    const bool col_ok = col < g.ncols;
-    if (!col_ok) wrow = 0;   // a valid row; its results are not stored
-    const uint8_t *row = M->data + (int64_t)e * M->mat_bytes + wrow * M->row_bytes;
-    const int64_t Kin = M->K;
-    if (tid < GB_BM) {
-        const int p = tid < mrows ? g.perm[start + tid] : -1;
-        s_p[tid] = p;
-        s_row[tid] = p < 0 ? 0 : (g.ne11 == 1 ? p / g.K : p);
-    }
-    __syncthreads();
-
-    // activation chunks of this thread: chunk q = tid + 256 i -> tile row q / 8, K chunk q % 8
-    uint4 areg[GB_ACH];
-    auto load_a = [&](int64_t k0) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < GB_ACH; ++i) {
-            const int q = tid + 256 * i, r = q >> 3, c = q & 7;
-            const int64_t k = k0 + 8 * c;
-            areg[i] = (r < 32 * nrt && k < Kin) ? *(const uint4 *)(g.xh + (int64_t)s_row[r] * Kin + k)
-                                               : make_uint4(0, 0, 0, 0);
-        }
-    };
-    auto store_a = [&](int buf) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < GB_ACH; ++i) {
-            const int q = tid + 256 * i, r = q >> 3, c = q & 7;
-            *(uint4 *)(&As[buf][(r * 8 + (c ^ (r & 7))) * 8]) = areg[i];
-        }
-    };
-
-    f32x16 acc[GB_RT];
-#pragma unroll
-    for (int t = 0; t < GB_RT; ++t)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) acc[t][i] = 0.f;
-
-    const int nk = (int)((Kin + GB_BK - 1) / GB_BK);
-    GBRaw<WT> cur, nxt;
-    load_a(0);
-    gb_load<WT>(row, 0, Kin, h, cur);
-    store_a(0);
-    __syncthreads();
-    for (int kb = 0; kb < nk; ++kb) {
-        const bool more = kb + 1 < nk;
-        if (more) {
-            load_a((int64_t)(kb + 1) * GB_BK);
-            gb_load<WT>(row, (int64_t)(kb + 1) * GB_BK, Kin, h, nxt);
-        }
-        const _Float16 *A = As[kb & 1];
-        auto step = [&](const half8_t bop, int s) __attribute__((always_inline)) {
-            const int c = 2 * s + h;
-#pragma unroll
-            for (int t = 0; t < GB_RT; ++t) {
-                if (t < nrt) {
-                    const int r = 32 * t + l32;
-                    const half8_t aop = *(const half8_t *)(&A[(r * 8 + (c ^ (r & 7))) * 8]);
-                    acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(aop, bop, acc[t], 0, 0, 0);
-                }
-            }
-        };
-        step(gb_operand<WT, 0>(cur, h), 0);
-        step(gb_operand<WT, 1>(cur, h), 1);
-        step(gb_operand<WT, 2>(cur, h), 2);
-        step(gb_operand<WT, 3>(cur, h), 3);
-        if (more) {
-            store_a((kb + 1) & 1);
-            cur = nxt;
-        }
-        __syncthreads();
-    }
-
-    // rows 32 t + 8 (i / 4) + 4 h + i % 4, column col
-    if (GLU) {
-        float *G = (float *)&As[0][0];   // [GB_BM][64] up-product values (48 KB)
-        const int cc = 32 * (wave & 1) + l32;
-        if (wave >= 2) {
-#pragma unroll
-            for (int t = 0; t < GB_RT; ++t)
-                if (t < nrt)
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) G[(32 * t + 8 * (i >> 2) + 4 * h + (i & 3)) * 64 + cc] = acc[t][i];
-        }
-        __syncthreads();
-        if (wave < 2 && col_ok) {
-#pragma unroll
-            for (int t = 0; t < GB_RT; ++t)
-                if (t < nrt)
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) {
-                        const int m = 32 * t + 8 * (i >> 2) + 4 * h + (i & 3);
-                        if (m < mrows) g.y[(int64_t)s_p[m] * g.ldy + col] = act_pair(g.act, acc[t][i], G[m * 64 + cc]);
-                    }
-        }
-    } else if (col_ok) {
-#pragma unroll
-        for (int t = 0; t < GB_RT; ++t)
-            if (t < nrt)
-#pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    const int m = 32 * t + 8 * (i >> 2) + 4 * h + (i & 3);
-                    if (m < mrows) g.y[(int64_t)s_p[m] * g.ldy + col] = acc[t][i];
-                }
-    }
-}
-
 // ------------------------------------------------------------------ launch
-template <template <int> class KF>
-static int b32_dispatch_type(int type, dim3 grid, const B32Args &g, hipStream_t st);
-
 int launch_gemv_b32(const B32Args &g, hipStream_t st) {
     if (g.max_active <= 0) return 0;
     if (g.a.K % 32) return -6;
@@ -517,24 +318,6 @@ int launch_gemv_b32(const B32Args &g, hipStream_t st) {
     case 8: hipLaunchKernelGGL(k_gemv_b32<8>, grid, dim3(256), 0, st, g); break;
     default: return -3;
     }
-    return hip_check_launch();
-}
-
-int launch_gemm_b32(const B32Args &g, hipStream_t st) {
-    if (g.max_tiles <= 0) return 0;
-    if (g.a.K % 32) return -6;
-    const dim3 grid((unsigned)(g.glu ? (g.ncols + 63) / 64 : (g.ncols + 127) / 128), (unsigned)g.max_tiles);
-#define GB_LAUNCH(T)                                                                                    \
-    if (g.glu) hipLaunchKernelGGL((k_gemm_b32<T, true>), grid, dim3(256), 0, st, g);                   \
-    else hipLaunchKernelGGL((k_gemm_b32<T, false>), grid, dim3(256), 0, st, g);
-    switch (g.a.type) {
-    case 1: GB_LAUNCH(1) break;
-    case 2: GB_LAUNCH(2) break;
-    case 6: GB_LAUNCH(6) break;
-    case 8: GB_LAUNCH(8) break;
-    default: return -3;
-    }
-#undef GB_LAUNCH
     return hip_check_launch();
 }
 

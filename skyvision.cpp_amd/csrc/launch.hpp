@@ -255,7 +255,8 @@ struct B32Prep {
                                // (their GEMM); F16: fp16(x) rows (F16 tables, both paths)
     int8_t *q8 = nullptr;      // CODES: [rows][K]
     uint16_t *dh = nullptr;    // CODES: [rows][K/32] fp16 scale bits
-    _Float16 *xh = nullptr;    // DQ / F16: [rows][K]
+    _Float16 *xh = nullptr;    // DQ / F16: [rows][ldo]
+    int64_t ldo = 0;           // >= K; values K .. ldo - 1 of a row are written as zeros
     int pre_act = 0;           // 4 (ACT_RELU_SQR): relu(v)^2 first
 };
 int launch_prep_b32(const float *src, int64_t ld, int64_t nrows, int64_t K, const B32Prep &o, hipStream_t st);
@@ -263,19 +264,44 @@ struct B32Args {
     ExpertMat a, b;            // b: up table (separate gate/up GLU), else unused
     int glu, fused, act;
     int64_t I;
-    const int8_t *q8;          // GEMV of Q4_0/Q5_0/Q8_0: Q8_0 codes [rows][K] and
+    const int8_t *q8;          // Q4_0/Q5_0/Q8_0: Q8_0 codes [rows][K] and
     const uint16_t *dh;        //   fp16 scales [rows][K/32]
-    const _Float16 *xh;        // GEMM (and F16 GEMV): fp16 rows [rows][K]
+    const _Float16 *xh;        // F16: fp16 rows [rows][K]
     int ne11, K;
-    const int32_t *counts, *offsets, *perm, *active_e, *n_active;   // GEMV
+    const int32_t *counts, *offsets, *perm, *active_e, *n_active;
     int max_active;
-    const int32_t *tile_e, *tile_start, *tile_rows, *n_tiles;       // GEMM: balanced tiles of G4_BM rows
-    int max_tiles;
     float *y;                  // rows p (glu: act rows [p][I]), stride ldy
     int64_t ldy, ncols;
 };
 int launch_gemv_b32(const B32Args &g, hipStream_t st);
-int launch_gemm_b32(const B32Args &g, hipStream_t st);
+
+// Grouped MFMA GEMM of the same tables (k_gb.hip) on balanced tiles of at
+// most bm rows.  xh: fp16 activation rows [xrows][ldx], ldx a multiple of 64,
+// zeros past K.  Plain product: fp32 rows y.  glu / relu_sqr: the
+// activation rows leave as the next product's operand xo [p][ldo] (ldo =
+// ncols rounded up to 64, zeros past ncols; ncols % 32 == 0): fp16(v), or
+// their Q8_0 as fp16(d q), the bits of launch_prep_b32 on the fp32 values.
+struct GBArgs {
+    ExpertMat a, b;            // b: up table (separate gate/up GLU), else unused
+    int glu, fused, act;
+    int relu_sqr;              // one product, relu(v)^2 of it
+    int64_t I;
+    const _Float16 *xh;
+    int64_t ldx, xrows;
+    uint32_t xbytes;           // (set by launch_gb)
+    int ne11, K;
+    const int32_t *perm, *tile_e, *tile_start, *tile_rows, *n_tiles;
+    int max_tiles, bm, nct;    // nct: column tiles (set by launch_gb)
+    float *y;
+    int64_t ldy, ncols;
+    _Float16 *xo;
+    int64_t ldo;
+    int next_f16;
+};
+constexpr int GB_BM_SMALL = 32, GB_BM_LARGE = 128;
+constexpr int64_t GB_MAX_X = 0xF0000000ll;          // bytes of xh (32-bit buffer offsets)
+constexpr int64_t GB_MAX_ROW_BYTES = 1ll << 25;
+int launch_gb(const GBArgs &g, hipStream_t st);
 
 // Single-token MoE block in one kernel (k_decode.hip).
 struct DecArgs {

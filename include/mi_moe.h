@@ -406,9 +406,9 @@ int mi_moe_ctx_set_gemm_threshold(mi_moe_ctx *ctx, int64_t min_tokens_for_gemm);
  * work-group per CU, the weight stream held in registers a group of blocks
  * ahead) on layers whose tables are all Q4_K with n_embd and n_ff <= 2048
  * (others take the shape rule); 4 8-row tiles wherever they apply (else
- * 32-row); 5 64-row tiles at every size.  Kinds 0-2, 4 and 5 give the same
- * bits (the same per-row
- * arithmetic); the skinny products sum each output's products in another
+ * 32-row); 5 64-row tiles at every size.  Q6_K gate/up layers have the 32-
+ * and 192-row tiles (kinds 2 and 4: 32-row; 1 and 5: 192-row).  Kinds 0-2, 4
+ * and 5 give the same bits (the same per-row arithmetic); the skinny products sum each output's products in another
  * order (fp32; the rows agree to ~2e-4 rel-L2 after the activations' fp16
  * and Q8_K roundings). */
 int mi_moe_ctx_set_gemm_tiles(mi_moe_ctx *ctx, int kind);

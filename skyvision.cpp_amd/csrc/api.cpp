@@ -423,9 +423,18 @@ bool use_gemm_wide(const mi_moe_ctx *c, int64_t T, int K, int E) {
 bool gemm_path(const mi_moe_ctx *c, const mi_moe_layer *L, int64_t T) {
     return use_gemm(c, T, L->n_expert_used, L->n_expert) || L->n_embd > 8 * QK || L->n_ff > 8 * QK;
 }
-// the 4-wave 32x32x16 GEMMs (Q4_K gate/up GLU, and every one-product layer);
-// else the 16x16x32 GEMM with its fused GLU + Q8_K epilogue (Q6_K gate/up)
-bool g4_path(const mi_moe_layer *L) { return L->gate.type == MI_TYPE_Q4_K || !act_gated(L->act); }
+// the 4-wave 32x32x16 GEMMs; else (Q6_K gate/up tables they do not take: gate
+// and up strides that differ, or activation rows past their 32-bit offsets)
+// the 16x16x32 GEMM with its fused GLU + Q8_K epilogue
+bool g4_path(const mi_moe_layer *L, int64_t T) {
+    if (L->gate.type == MI_TYPE_Q4_K || !act_gated(L->act)) return true;
+    const int64_t lim = 0x7fffffff, rows = T * L->n_expert_used;
+    if (T * L->n_embd * 2 > lim || rows * L->n_ff * 2 > lim) return false;
+    if ((int64_t)L->gate.nb[2] + 4 > lim || (int64_t)L->down.nb[2] + 4 > lim) return false;
+    if (L->fused_gate_up) return true;
+    const ExpertMat up = as_mat(L->up);
+    return (int64_t)L->up.nb[2] + 4 <= lim && g4_q6k_glu_ok(as_mat(L->gate), &up);
+}
 
 // Row tiles of the 4-wave GEMMs: 32-row tiles (52 KB of LDS with Q4_K
 // weights: three work-groups per CU keep more of the weight stream in flight) when the call
@@ -523,7 +532,7 @@ bool x_q8_spec(const mi_moe_ctx *c, const mi_moe_layer *L, int64_t T, Q8Out &qx)
     if (!gemm_path(c, L, T)) {
         qx.q8 = c->ax.q8; qx.d8 = c->ax.d8; qx.bsums = c->ax.bs;
     } else {
-        qx.xh = c->ax.h; qx.wtype = L->gate.type; qx.order = g4_path(L) ? 1 : 0;
+        qx.xh = c->ax.h; qx.wtype = L->gate.type; qx.order = g4_path(L, T) ? 1 : 0;
         qx.range_total = c->range_total;
     }
     return true;
@@ -664,9 +673,12 @@ int run_experts(mi_moe_ctx *c, const mi_moe_layer *L, const float *x, int64_t T,
     const bool gemm = kq && gemm_path(c, L, T);
     // GEMM M-tiles: balanced tiles of at most G4_BM rows for the 4-wave GEMMs,
     // GEMM_BM-row tiles otherwise
-    const bool g4 = gemm && g4_path(L);
+    const bool g4 = gemm && g4_path(L, T);
+    // Q6_K gate/up: the GLU rows and the slot rows stay fp32
+    const bool rows32 = gated && L->gate.type == MI_TYPE_Q6_K;
     const bool gs = g4 && gs_path(c, L, T);
-    const int bm = !g4 ? GEMM_BM : gs ? GS_BM : g4_small_tiles(c, L, T) ? G4_BM_SMALL : g4_mid_tiles(c, L, T) ? G4_BM_MID : G4_BM;
+    const int bm = !g4 ? GEMM_BM : gs ? GS_BM : g4_small_tiles(c, L, T) ? G4_BM_SMALL :
+                   !rows32 && g4_mid_tiles(c, L, T) ? G4_BM_MID : G4_BM;   // (Q6_K gate/up: LDS for one work-group either way)
     const int max_tiles = (int)((rows + bm - 1) / bm + max_active);
     // Small calls on the 32-row tiles, ids from the router: no dispatch
     // launch, each GEMM work-group finds its tile from the ids itself
@@ -678,7 +690,7 @@ int run_experts(mi_moe_ctx *c, const mi_moe_layer *L, const float *x, int64_t T,
                            E <= 256;
     // without a dispatch, each product may take 8-row tiles (its own tiles
     // from the ids; the tile tables are not used)
-    const bool tiny = self_disp && g4_tiny_tiles(c, L, T);
+    const bool tiny = self_disp && !rows32 && g4_tiny_tiles(c, L, T);
     const int bm_gu = tiny ? G4_BM_TINY : bm;
     const int bm_dn = tiny && L->down.type == MI_TYPE_Q4_K ? G4_BM_TINY : bm;
     if (!self_disp) {
@@ -782,18 +794,18 @@ int run_experts(mi_moe_ctx *c, const mi_moe_layer *L, const float *x, int64_t T,
         a.y = c->f1; a.ldy = I; a.ncols = I; a.xrows = T;
         // gated: the GLU rows as fp16 (half the bytes of their round trip to
         // the Q8_K pass; saturation at the fp16 range is counted)
-        if (gated) { a.yh = (_Float16 *)c->f1; a.range_total = c->range_total; }
+        if (gated && !rows32) { a.yh = (_Float16 *)c->f1; a.range_total = c->range_total; }
         if (!gs) prof_clock(c, a, 0);   // (the skinny kernels record no clocks)
         TRY(gs ? launch_gemm_gs(a, gs_splits(c, rows, E, gated ? I : a.ncols, a.glu), st) : launch_gemm4(a, st));
         stage_end(c, "gate_up", st);
-        // the 32-row down product quantizes its own rows (gated: fp16 GLU rows)
+        // the 32-row down product quantizes its own rows (gated)
         const bool own_q8 = bm_dn <= G4_BM_SMALL && !gs && gated;
         Q8Out qa;
         qa.xh = c->aact.h; qa.wtype = down.type; qa.order = 1; qa.pre_act = gated ? 0 : MI_ACT_RELU_SQR;
         qa.range_total = c->range_total;
         if (own_q8) {
             // (no pass: the down product's work-groups quantize their rows)
-        } else if (gated) {
+        } else if (gated && !rows32) {
             TRY(launch_q8k_rows((const _Float16 *)c->f1, I, rows, I, qa, st));
         } else {
             TRY(launch_q8k_rows(c->f1, I, rows, I, qa, st));
@@ -802,7 +814,11 @@ int run_experts(mi_moe_ctx *c, const mi_moe_layer *L, const float *x, int64_t T,
         G2Args d = {};
         d.a = down; d.glu = 0; d.xh = c->aact.h; d.ne11 = K; d.K = K;
         if (L->down_tiled.data) { d.a = as_mat(L->down_tiled); d.tiled = 1; }
-        if (own_q8) { d.q8src = (const _Float16 *)c->f1; d.q8ld = I; }
+        if (own_q8) {
+            if (rows32) d.q8src32 = c->f1;
+            else d.q8src = (const _Float16 *)c->f1;
+            d.q8ld = I;
+        }
         d.counts = dd.counts; d.offsets = dd.offsets; d.perm = dd.perm; d.tile_e = dd.tile_e;
         d.tile_r0 = dd.tile_r0; d.tile_start = dd.tile_start; d.tile_rows = dd.tile_rows; d.n_tiles = dd.n_tiles; d.max_tiles = max_tiles; d.xrows = (int64_t)T * K;
         d.tile_perm = dd.tile_perm;
@@ -813,12 +829,13 @@ int run_experts(mi_moe_ctx *c, const mi_moe_layer *L, const float *x, int64_t T,
         }
         // the slot rows as fp16 (half the bytes of the round trip to the
         // combine; saturation at the fp16 range is counted)
-        d.y = c->z; d.yh = zh = (_Float16 *)c->z; d.range_total = c->range_total; d.ldy = D; d.ncols = D;
+        d.y = c->z; d.range_total = c->range_total; d.ldy = D; d.ncols = D;
+        if (!rows32) d.yh = zh = (_Float16 *)c->z;
         if (!gs) prof_clock(c, d, 1);
         TRY(gs ? launch_gemm_gs(d, gs_splits(c, rows, E, D, 0), st) : launch_gemm4(d, st));
         stage_end(c, "down", st);
     } else {
-        // Q6_K gate/up: fp16 dequant on 16x16x32 MFMA
+        // Q6_K gate/up past the 4-wave GEMMs: fp16 dequant on 16x16x32 MFMA
         GemmArgs a = {};
         a.a = gate; a.b = up; a.epi = EPI_GLU; a.act = L->act; a.I = I; a.fused = L->fused_gate_up;
         a.xh = c->ax.h; a.ne11 = 1; a.K = K;

@@ -1,4 +1,6 @@
-// k_gemm.hip - grouped k-quant GEMM on fp16 MFMA for prefill.
+// k_gemm.hip - grouped k-quant GEMM on fp16 MFMA for prefill: the layers with
+// Q6_K gate/up tables that the 4-wave GEMMs (k_gemm4.hip) do not take (gate
+// and up strides that differ, activation rows past 32-bit offsets).
 //
 // One work-group computes a 64-row tile of one expert's token list (rows are
 // the dispatched (token, slot) pairs, gathered through the permutation) against
@@ -324,9 +326,8 @@ int launch_gemm(const GemmArgs &g, hipStream_t st) {
     const dim3 grid(gx, (unsigned)g.max_tiles);
     const dim3 block(GM_THREADS);
     if (g.a.type == 12) {
-        if (!glu) hipLaunchKernelGGL((k_gemm<12, false, 12>), grid, block, 0, st, g);
-        else if (g.next_type == 14) hipLaunchKernelGGL((k_gemm<12, true, 14>), grid, block, 0, st, g);
-        else hipLaunchKernelGGL((k_gemm<12, true, 12>), grid, block, 0, st, g);
+        if (glu) return -3;   // (Q4_K gate/up: launch_gemm4)
+        hipLaunchKernelGGL((k_gemm<12, false, 12>), grid, block, 0, st, g);
     } else if (g.a.type == 14) {
         if (!glu) hipLaunchKernelGGL((k_gemm<14, false, 12>), grid, block, 0, st, g);
         else if (g.next_type == 14) hipLaunchKernelGGL((k_gemm<14, true, 14>), grid, block, 0, st, g);

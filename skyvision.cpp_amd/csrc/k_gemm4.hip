@@ -1,5 +1,5 @@
 // k_gemm4.hip - grouped k-quant GEMMs of the prefill on v_mfma_f32_32x32x16_f16:
-// gate/up with the GLU fused in (k_g4_glu, fp32 activations out) and the
+// gate/up with the GLU fused in (k_g4_glu) and the
 // plain product (k_g4_store: the down product, mul_mat_id).
 //
 // One work-group of 4 waves per CU, one wave per SIMD.  A work-group owns a
@@ -785,14 +785,19 @@ __device__ __forceinline__ void g4_clock(const G2Args &g, int slot, bool live) {
 // with Q4_K weights, so that three work-groups share a CU and keep three
 // times the weight stream in flight; G4_BM_TINY, calls without a dispatch
 // launch and at most 4 rows per expert: 40 KB, four work-groups per CU)
-template <int BM>
+// WT 14 (Q6_K gate/up): 32- and 192-row tiles (80 and 160 KB of LDS), fp32
+// GLU rows.  The layers that take it ran 64-row tiles of 16x16x32 MFMAs with
+// each lane loading its own weight rows (k_gemm): moondream3 T = 509, gate/up
+// with its Q8_K epilogue 218 -> 87 us + 6 us of Q8_K pass, down 104 -> 56 us,
+// the layer 356 -> 178 us.
+template <int WT, int BM>
 __global__ void __launch_bounds__(G4_THREADS)
-    __attribute__((amdgpu_waves_per_eu(BM == G4_BM_TINY ? 4 : BM == G4_BM_MID ? 2 : 1, BM == G4_BM ? 1 : BM == G4_BM_TINY ? 4 : BM == G4_BM_MID ? 2 : 3)))
+    __attribute__((amdgpu_waves_per_eu(BM == G4_BM_TINY ? 4 : BM == G4_BM_MID ? 2 : 1, BM == G4_BM ? 1 : BM == G4_BM_TINY ? 4 : BM == G4_BM_MID || WT == 14 ? 2 : 3)))
     k_g4_glu(G2Args g) {
     constexpr int NA = BM >= 32 ? BM / 32 : 1, TR = BM < 32 ? BM : 0;
     __shared__ __attribute__((aligned(1024))) _Float16 As0[BM * G4_SK];
     __shared__ __attribute__((aligned(1024))) _Float16 As1[BM * G4_SK];
-    __shared__ __attribute__((aligned(1024))) uint8_t Ws[G4_WAVES][g4_wregion<12>()];
+    __shared__ __attribute__((aligned(1024))) uint8_t Ws[G4_WAVES][g4_wregion<WT>()];
     int tile, ctile;
     g4_coords((int)(g.I / 128), tile, ctile);
     const bool self = BM <= G4_BM_SMALL && g.ids != nullptr;
@@ -811,19 +816,25 @@ __global__ void __launch_bounds__(G4_THREADS)
     // weight rows: h rows n0 .. n0 + 31 (column tile 0), g rows at I + n0 of
     // the fused matrix or n0 of the up matrix (column tile 1)
     const int64_t n0 = (int64_t)ctile * 128 + 32 * wave;
-    const rsrc_t ra = g4_rsrc(g.a.data + (int64_t)t.e * g.a.mat_bytes, g.a.mat_bytes);
-    const rsrc_t rg = g.fused ? ra : g4_rsrc(g.b.data + (int64_t)t.e * g.b.mat_bytes, g.b.mat_bytes);
+    // (Q6_K: both matrices start the same number of bytes past a dword, as do
+    // the rows of both column tiles; the launch checks it)
+    const uint8_t *ma = g.a.data + (int64_t)t.e * g.a.mat_bytes;
+    const uint8_t *mb = g.fused ? ma : g.b.data + (int64_t)t.e * g.b.mat_bytes;
+    const uint32_t mis = WT == 14 ? (uint32_t)((uintptr_t)ma & 3u) : 0u;
+    const uint32_t rb = (uint32_t)g.a.row_bytes;
+    const rsrc_t ra = g4_rsrc(ma - mis, g.a.mat_bytes + mis);
+    const rsrc_t rg = g.fused ? ra : g4_rsrc(mb - mis, g.b.mat_bytes + mis);
     const int64_t rowbase[2] = {n0, g.fused ? g.I + n0 : n0};
-    const G4WDma<12> dm = g4_wdma<12>(ra, rg, rowbase, (uint32_t)g.a.row_bytes, 0u, lane, g.tiled != 0);
-    g4_issue_w0<12>(dm, Ws[wave]);
+    const G4WDma<WT> dm = g4_wdma<WT>(ra, rg, rowbase, rb, mis, lane, WT == 12 && g.tiled != 0);
+    g4_issue_w0<WT>(dm, Ws[wave]);
     // the activation rows live in the second activation buffer until the K
     // loop has computed its load offsets (its first write comes later)
     int *s_arow = (int *)As1;
     g4_rows_publish<BM>(g, my_p, s_arow);
-    const uint32_t wsh[2] = {0u, 0u};
+    const uint32_t ws0 = mis + (uint32_t)(n0 + (lane & 31)) * rb, wsh[2] = {ws0, ws0};   // (Q6_K block alignment)
     f32x16 acc[NA][2];
     u32x4 sn[2];   // (Q6_K tiled only)
-    g4_kloop<12, NA, TR>(rx, s_arow, 2u * Kin, dm, wsh, Ws[wave], (int)(Kin / QK), wave, lane, nrt, As0, As1, acc, sn);
+    g4_kloop<WT, NA, TR>(rx, s_arow, 2u * Kin, dm, wsh, Ws[wave], (int)(Kin / QK), wave, lane, nrt, As0, As1, acc, sn);
     __builtin_amdgcn_s_waitcnt(0);   // no load may land in LDS after the work-group ends
     const int *s_p = g4_publish_rows<BM>((_Float16 *)&Ws[0][0], my_p);   // the row table in the weight region
     switch (g.act) {
@@ -853,7 +864,8 @@ __device__ __forceinline__ void g4_q8_rows(const G2Args &g, int mrows, const int
         const int64_t p = s_arow[r];
         float v[16];
         if (bok) {
-            q8h_gather<XO>(g.q8src + p * g.q8ld + (int64_t)b * QK, s, v);
+            if (g.q8src) q8h_gather<XO>(g.q8src + p * g.q8ld + (int64_t)b * QK, s, v);
+            else q8h_gather<XO>(g.q8src32 + p * g.q8ld + (int64_t)b * QK, s, v);
         } else {
 #pragma unroll
             for (int i = 0; i < 16; ++i) v[i] = 0.f;
@@ -908,7 +920,7 @@ __global__ void __launch_bounds__(G4_THREADS)
     int *s_arow = (int *)As1;   // as in k_g4_glu
     g4_rows_publish<BM>(g, my_p, s_arow);
     if constexpr (BM <= G4_BM_SMALL) {
-        if (g.q8src) g4_q8_rows<WT == 12 ? XO_Q4 : XO_Q6>(g, t.mrows, s_arow, ctile == 0, wave, lane);
+        if (g.q8src || g.q8src32) g4_q8_rows<WT == 12 ? XO_Q4 : XO_Q6>(g, t.mrows, s_arow, ctile == 0, wave, lane);
     }
     // byte offset of the lane's own rows (Q6_K block alignment)
     const uint32_t wsh[2] = {mis + (uint32_t)(n0 + l32) * rb, mis + (uint32_t)(n0 + 32 + l32) * rb};
@@ -973,6 +985,13 @@ int gemm4_grid(const G2Args &g) {
     return 8 * nct * ntile8;
 }
 
+// One byte shift serves a lane's gate and up rows of a Q6_K block: equal row
+// strides, and matrices that start equally far past a dword for every expert.
+bool g4_q6k_glu_ok(const ExpertMat &a, const ExpertMat *b) {
+    return !b || (a.row_bytes == b->row_bytes && ((uintptr_t)a.data - (uintptr_t)b->data) % 4 == 0 &&
+                  (a.mat_bytes - b->mat_bytes) % 4 == 0);
+}
+
 int launch_gemm4(const G2Args &g, hipStream_t st) {
     if (g.max_tiles <= 0) return 0;
     if (g.a.K % QK) return -6;
@@ -994,23 +1013,31 @@ int launch_gemm4(const G2Args &g, hipStream_t st) {
                     (g.glu && !g.fused &&
                      (g.b.type != 12 || g.b.N % 32 || g.b.mat_bytes != g.b.N * g.b.row_bytes))))
         return -6;
-    if (g.q8src && (g.glu || g.bm > G4_BM_SMALL || g.q8ld % 4 || (uintptr_t)g.q8src % 8 || (uintptr_t)g.xh % 16))
+    if ((g.q8src || g.q8src32) && (g.glu || g.bm > G4_BM_SMALL || g.q8ld % 4 || (uintptr_t)g.q8src % 8 ||
+                                   (uintptr_t)g.q8src32 % 16 || (uintptr_t)g.xh % 16))
         return -6;
     const int ntile8 = (g.max_tiles + 7) / 8;
     if (g.glu) {
         // GLU values out (fp32 to y or fp16 to yh, ldy); the work-group covers
         // 128 act columns
-        if (g.a.type != 12 || (g.I % 128)) return -6;
+        if ((g.a.type != 12 && g.a.type != 14) || (g.I % 128)) return -6;
         if (g.yh ? (g.ldy % 8 || (uintptr_t)g.yh % 16) : (g.ldy % 4 || (uintptr_t)g.y % 16)) return -6;
-        if (!g.fused && (g.b.mat_bytes > lim || g.b.type != 12 || g.b.row_bytes != g.a.row_bytes)) return -6;
-        if ((uintptr_t)g.a.data % 4 || g.a.mat_bytes % 4 || g.a.row_bytes % 4) return -6;
-        if (!g.fused && ((uintptr_t)g.b.data % 4 || g.b.mat_bytes % 4)) return -6;
+        if (!g.fused && (g.b.mat_bytes + 4 > lim || g.b.type != g.a.type || g.b.row_bytes != g.a.row_bytes)) return -6;
         const int nct = (int)(g.I / 128);
         const dim3 grid((unsigned)(8 * nct * ntile8));
-        if (g.bm == G4_BM_TINY) hipLaunchKernelGGL(k_g4_glu<G4_BM_TINY>, grid, dim3(G4_THREADS), 0, st, g);
-        else if (g.bm == G4_BM_SMALL) hipLaunchKernelGGL(k_g4_glu<G4_BM_SMALL>, grid, dim3(G4_THREADS), 0, st, g);
-        else if (g.bm == G4_BM_MID) hipLaunchKernelGGL(k_g4_glu<G4_BM_MID>, grid, dim3(G4_THREADS), 0, st, g);
-        else hipLaunchKernelGGL(k_g4_glu<G4_BM>, grid, dim3(G4_THREADS), 0, st, g);
+        if (g.a.type == 14) {
+            if (!g4_q6k_glu_ok(g.a, g.fused ? nullptr : &g.b)) return -6;
+            if (g.bm == G4_BM_SMALL) hipLaunchKernelGGL((k_g4_glu<14, G4_BM_SMALL>), grid, dim3(G4_THREADS), 0, st, g);
+            else if (g.bm == G4_BM) hipLaunchKernelGGL((k_g4_glu<14, G4_BM>), grid, dim3(G4_THREADS), 0, st, g);
+            else return -6;
+            return hip_check_launch();
+        }
+        if ((uintptr_t)g.a.data % 4 || g.a.mat_bytes % 4 || g.a.row_bytes % 4) return -6;
+        if (!g.fused && ((uintptr_t)g.b.data % 4 || g.b.mat_bytes % 4)) return -6;
+        if (g.bm == G4_BM_TINY) hipLaunchKernelGGL((k_g4_glu<12, G4_BM_TINY>), grid, dim3(G4_THREADS), 0, st, g);
+        else if (g.bm == G4_BM_SMALL) hipLaunchKernelGGL((k_g4_glu<12, G4_BM_SMALL>), grid, dim3(G4_THREADS), 0, st, g);
+        else if (g.bm == G4_BM_MID) hipLaunchKernelGGL((k_g4_glu<12, G4_BM_MID>), grid, dim3(G4_THREADS), 0, st, g);
+        else hipLaunchKernelGGL((k_g4_glu<12, G4_BM>), grid, dim3(G4_THREADS), 0, st, g);
     } else {
         const int nct = (int)((g.ncols + G4_NWG - 1) / G4_NWG);
         const dim3 grid((unsigned)(8 * nct * ntile8));

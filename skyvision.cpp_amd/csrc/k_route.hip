@@ -419,8 +419,7 @@ __global__ void __launch_bounds__(1024) k_front(const float *__restrict__ W, con
             if (row >= T) continue;
             int8_t *sq = (int8_t *)stg;
             float *sd = (float *)(stg + 64);
-            if (XO == XO_Q4) q8k_row_group<VEC, XO_Q4>(x, ldx, row, i % ngrp, nb, o, sq, sd, lane);
-            else q8k_row_group<VEC, XO_ANY>(x, ldx, row, i % ngrp, nb, o, sq, sd, lane);
+            q8k_row_group<VEC, XO>(x, ldx, row, i % ngrp, nb, o, sq, sd, lane);
         }
     }
     __syncthreads();
@@ -495,8 +494,7 @@ __global__ void __launch_bounds__(1024) k_front_parts(const float *__restrict__ 
             if (row >= T) continue;
             int8_t *sq = (int8_t *)stg;
             float *sd = (float *)(stg + 64);
-            if (XO == XO_Q4) q8k_row_group<VEC, XO_Q4>(x, ldx, row, i % ngrp, nb, o, sq, sd, lane);
-            else q8k_row_group<VEC, XO_ANY>(x, ldx, row, i % ngrp, nb, o, sq, sd, lane);
+            q8k_row_group<VEC, XO>(x, ldx, row, i % ngrp, nb, o, sq, sd, lane);
         }
     }
 }
@@ -514,6 +512,9 @@ int launch_front(const float *W, const float *b, const float *x, int64_t ldx, in
     const Q8Out o = qx ? *qx : Q8Out{};
     if (vec && q8_xo(o) == XO_Q4)
         hipLaunchKernelGGL((k_front<true, XO_Q4>), dim3((unsigned)blocks), dim3(64 * RT_WAVES), 0, st, W, b, x, ldx,
+                           T, D, E, logits, o);
+    else if (vec && q8_xo(o) == XO_Q6)
+        hipLaunchKernelGGL((k_front<true, XO_Q6>), dim3((unsigned)blocks), dim3(64 * RT_WAVES), 0, st, W, b, x, ldx,
                            T, D, E, logits, o);
     else if (vec)
         hipLaunchKernelGGL((k_front<true, XO_ANY>), dim3((unsigned)blocks), dim3(64 * RT_WAVES), 0, st, W, b, x,
@@ -538,6 +539,8 @@ int launch_front_parts(const float *W, const float *x, int64_t ldx, int64_t T, i
     const dim3 grid((unsigned)blocks), block((unsigned)(64 * cps));
     if (vec && q8_xo(o) == XO_Q4)
         hipLaunchKernelGGL((k_front_parts<true, XO_Q4>), grid, block, 0, st, W, x, ldx, T, D, E, cps, parts, o);
+    else if (vec && q8_xo(o) == XO_Q6)
+        hipLaunchKernelGGL((k_front_parts<true, XO_Q6>), grid, block, 0, st, W, x, ldx, T, D, E, cps, parts, o);
     else if (vec)
         hipLaunchKernelGGL((k_front_parts<true, XO_ANY>), grid, block, 0, st, W, x, ldx, T, D, E, cps, parts, o);
     else

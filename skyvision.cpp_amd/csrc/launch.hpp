@@ -172,7 +172,8 @@ int launch_gemm(const GemmArgs &g, hipStream_t st);
 // 4-wave grouped GEMMs on 32x32x16 MFMA (k_gemm4.hip), tiles of at most
 // G4_BM rows from a balanced dispatch.  Both take fp16 activations in the
 // weight type's 32x32x16 MFMA K order (xh; xd, xbs, acth and next_type are
-// not read).  glu = 1: Q4_K gate/up (fused [h | g] or separate), writes the
+// not read).  glu = 1: Q4_K or Q6_K gate/up (fused [h | g] or separate; Q6_K:
+// bm = G4_BM or G4_BM_SMALL, tables that g4_q6k_glu_ok takes), writes the
 // GLU rows (fp32 to y or fp16 to yh, ldy), whose Q8_K the caller computes
 // (launch_q8k_rows) for the down product; glu = 0: Q4_K / Q6_K product, rows
 // to y (fp32) or yh (fp16).
@@ -203,6 +204,7 @@ struct G2Args {
     // bits the separate Q8_K pass writes (work-groups of column tile 0 count
     // its saturations)
     const _Float16 *q8src;
+    const float *q8src32;   // the same from fp32 rows (q8src NULL)
     int64_t q8ld;
     // 1: a (and b) hold tables in the tiled order (launch_tile_q4k: the 32
     // rows of a column tile give block b as 4608 contiguous bytes, the LDS
@@ -230,6 +232,7 @@ constexpr int G4_BM_SMALL = 32;   // tiles of few rows per expert (G2Args::bm)
 constexpr int G4_BM_MID = 64;     // two work-groups per CU (G2Args::bm; Q4_K weights)
 constexpr int G4_BM_TINY = 8;     // tiles of at most 8 rows (G2Args::bm; only with ids: no dispatch launch)
 constexpr int G4_SD_IDS = 1024;    // most ids of a call whose GEMM work-groups find their tiles themselves (G2Args::ids)
+bool g4_q6k_glu_ok(const ExpertMat &a, const ExpertMat *b);
 int launch_gemm4(const G2Args &g, hipStream_t st);
 int gemm4_grid(const G2Args &g);   // work-groups launch_gemm4 launches
 

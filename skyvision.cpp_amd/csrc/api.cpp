@@ -287,22 +287,23 @@ int validate_layer(const mi_moe_ctx *c, const mi_moe_layer *L, bool need_router,
 
 // Single-token fused kernel: shape and layout conditions, and the work split
 // (P (h, g) row pairs per WG for gate/up, C output columns per WG for down).
-bool plan_decode1(const mi_moe_ctx *c, const mi_moe_layer *L, const float *x, int &P, int &C) {
+// ids: its caller-routed form (no router, gating or shared expert in it).
+bool plan_decode1(const mi_moe_ctx *c, const mi_moe_layer *L, const float *x, int &P, int &C, bool ids = false) {
     const int64_t D = L->n_embd, E = L->n_expert, K = L->n_expert_used, I = L->n_ff;
     const int G = c->dec_grid;
     if (!c->fused_decode || G <= 0) return false;
     // the fused kernel ranks and weights with the default gating only, runs
     // gated experts and no shared expert
-    if (L->gating != MI_GATING_SOFTMAX_TOPK || L->expert_scale) return false;
-    if (!act_gated(L->act) || L->sh_n_ff > 0) return false;
+    if (!ids && (L->gating != MI_GATING_SOFTMAX_TOPK || L->expert_scale || L->sh_n_ff > 0)) return false;
+    if (!act_gated(L->act)) return false;
     if (L->gate.type != MI_TYPE_Q4_K || (!L->fused_gate_up && L->up.type != MI_TYPE_Q4_K)) return false;
     if (L->down.type != MI_TYPE_Q4_K && L->down.type != MI_TYPE_Q6_K) return false;
     if (D % QK || I % QK || K > 8 || E > 256) return false;
-    if (E > G || D / QK > E) return false;   // one router row per WG; x-quant WGs also route
+    if (!ids && (E > G || D / QK > E)) return false;   // one router row per WG; x-quant WGs also route
     const int64_t NB = D / QK, NBI = I / QK;
     if (!(NB == 1 || NB == 2 || NB == 4 || NB == 8) || NBI > 8) return false;
     auto al16 = [](const void *p) { return ((uintptr_t)p & 15) == 0; };
-    if (!al16(x) || !al16(L->router_w) || !al16(L->gate.data) || !al16(L->down.data)) return false;
+    if (!al16(x) || (!ids && !al16(L->router_w)) || !al16(L->gate.data) || !al16(L->down.data)) return false;
     if (L->gate.nb[2] % 16 || L->down.nb[2] % 16) return false;
     if (!L->fused_gate_up && (!al16(L->up.data) || L->up.nb[2] % 16)) return false;
     P = 0;
@@ -319,8 +320,10 @@ bool plan_decode1(const mi_moe_ctx *c, const mi_moe_layer *L, const float *x, in
 }
 
 int run_decode1(mi_moe_ctx *c, const mi_moe_layer *L, const float *x, const float *res, float *out, int P,
-                int C, const NormParams &np, hipStream_t st) {
+                int C, const NormParams &np, hipStream_t st, const int32_t *ids_gu = nullptr,
+                const int32_t *ids_dn = nullptr, const float *wts = nullptr) {
     DecArgs g = {};
+    g.ids_gu = ids_gu; g.ids_dn = ids_dn; g.wts = wts; g.bad_total = c->bad_total;
     g.rw = L->router_w; g.rb = L->router_b; g.x = x;
     g.D = L->n_embd; g.E = L->n_expert; g.K = L->n_expert_used; g.I = L->n_ff;
     g.gate = as_mat(L->gate);
@@ -1405,6 +1408,25 @@ int mi_moe_expert_ffn(mi_moe_ctx *c, const mi_moe_layer *L, const float *x, int6
     HIP_TRY(hipSetDevice(c->device));
     hipStream_t st = (hipStream_t)stream;
     stage_begin(c, st);
+    // One or two tokens on the fused kernel, a launch each (layer us against
+    // the chain: qwen3omni 16.2 / 29.4 at one, 32.8 / 35.5 at two, three
+    // tokens 48.7 / 45.7; moondream3 18.5 / 33 and 37 / 42), unless the caller
+    // asked for the GEMM at that size or out overlaps what every work-group of
+    // the kernel reads (a late one may read after others wrote their columns).
+    int P = 0, C = 0;
+    const int64_t D = L->n_embd, K = L->n_expert_used;
+    auto apart = [&](const void *p, int64_t n) {
+        const uintptr_t a = (uintptr_t)p, o = (uintptr_t)out;
+        return a + (uintptr_t)(4 * n) <= o || o + (uintptr_t)(4 * T * D) <= a;
+    };
+    if (T <= 2 && (c->gemm_threshold == 0 || T < c->gemm_threshold) && apart(x, T * D) && apart(gate_up_ids, T * K) &&
+        apart(down_ids, T * K) && apart(w, T * K) && (!res || res == out || T == 1 || apart(res, T * D)) &&
+        plan_decode1(c, L, x, P, C, true)) {
+        for (int64_t t = 0; t < T; ++t)
+            TRY(run_decode1(c, L, x + t * D, res ? res + t * D : nullptr, out + t * D, P, C, NormParams{}, st,
+                            gate_up_ids + t * K, down_ids + t * K, w + t * K));
+        return MI_MOE_OK;
+    }
     return run_experts(c, L, x, T, gate_up_ids, down_ids, w, res, out, st, false, true);
 }
 

@@ -23,6 +23,8 @@
 //      while the activations are handed over) and unpacks them into a
 //      dot-ready form.
 //   -- activations --
+//   (the caller-routed form, mi_moe_expert_ffn: no A and no ranking, every WG
+//   quantizes x itself)
 //   C  per WG: Q8_K of each slot's activations, down dots from the
 //      LDS-resident rows of its columns, weighted combine in slot order
 //      (fp64, ggml's sum_rows of the weighted rows) and residual add.
@@ -217,6 +219,19 @@ __device__ inline void dec_q8k_x(const DecArgs &g, int b, int lane, const float4
                 (uint32_t)(uint16_t)(int16_t)s | ((uint32_t)(uint16_t)(int16_t)s_hi << 16));
 }
 
+// Caller-routed form: Q8_K of x block b (this wave's values v of it) into the
+// work-group's own LDS copy: codes, then 16-value block sums, then scales.
+constexpr int DEC_XQ_BS = 8 * QK, DEC_XQ_D = DEC_XQ_BS + 2 * (8 * QK / 16);   // (D <= 2048)
+__device__ inline void dec_q8k_x_lds(const float4_t xv, uint8_t *xl, int b, int lane) {
+    const float v[4] = {xv[0], xv[1], xv[2], xv[3]};
+    int q[4];
+    const float d = q8k_wave(v, lane, q);
+    *(uint32_t *)(xl + b * QK + 4 * lane) = pack_i8x4(q);
+    const int s = q8k_bsum16(q);
+    if ((lane & 3) == 0) *(int16_t *)(xl + DEC_XQ_BS + 2 * (b * 16 + (lane >> 2))) = (int16_t)s;
+    if (lane == 0) *(float *)(xl + DEC_XQ_D + 4 * b) = d;
+}
+
 // Sum of the NORM_T partials held by threads T0 .. T0 + NORM_T - 1 of the WG
 // (v of the others is ignored), paired as k_norm_rows pairs them: red[t] +=
 // red[t + o] for o = NORM_T / 2 .. 1 (two levels through LDS, the rest by lane
@@ -331,6 +346,17 @@ __device__ inline Q4X dec_q4x_load(const int8_t *xq, const int16_t *xbs, const f
     x.bsa = (int)(int16_t)(uint16_t)(wa >> sh);
     x.bsb = (int)(int16_t)(uint16_t)(wb >> sh);
     x.dx = __builtin_bit_cast(float, co_ld4(rd, 4u * (uint32_t)b));
+    return x;
+}
+// (from the work-group's own copy, dec_q8k_x_lds)
+__device__ inline Q4X dec_q4x_lds(const uint8_t *xl, int b, int sl) {
+    const int c = sl >> 1, l0 = 16 * (sl & 1);
+    Q4X x;
+    x.xa = *(const u32x4 *)(xl + b * QK + 64 * c + l0);
+    x.xb = *(const u32x4 *)(xl + b * QK + 64 * c + 32 + l0);
+    x.bsa = *(const int16_t *)(xl + DEC_XQ_BS + 2 * (b * 16 + 4 * c + (sl & 1)));
+    x.bsb = *(const int16_t *)(xl + DEC_XQ_BS + 2 * (b * 16 + 4 * c + 2 + (sl & 1)));
+    x.dx = *(const float *)(xl + DEC_XQ_D + 4 * b);
     return x;
 }
 __device__ inline float dec_q4_piece(const uint8_t *blk, int sl, const Q4X &x) {
@@ -509,17 +535,24 @@ __device__ inline DecChunk dec_chunk(const ExpertMat &m, int e, int64_t row0, in
 constexpr int DEC_RSTEPS = 16;   // row steps per wave in the gate/up phase (R / RPS)
 
 // NBI = I / 256: blocks per down row (compile time, so the per-slot Q8_K and
-// the down reductions unroll)
-template <int DT, int NBI>
+// the down reductions unroll).  IDS: the caller's expert ids and weights
+// (DecArgs::ids_gu ..) in place of phase A - no router, no ranking and no
+// hand-off of x: every work-group quantizes x itself (one block per wave)
+// behind its weight loads, which the ids alone place, so they go out at once.
+// Bound by the latency of its loads and of the one hand-off of the
+// activations.  qwen3omni, T = 1: the chain's six launches 29.4 us per call,
+// this kernel 16.2 us.
+template <int DT, int NBI, bool IDS>
 __global__ void __launch_bounds__(DEC_THREADS) k_decode1(DecArgs g) {
     __shared__ __attribute__((aligned(1024))) uint8_t s_gu[DEC_WAVES][DEC_WREG];
     __shared__ __attribute__((aligned(1024))) uint8_t s_dn[DEC_KMAX][DEC_DN_SEG * 1024];
     __shared__ float s_logit[256];
     __shared__ int s_sel[DEC_KMAX];
     __shared__ float s_val[DEC_KMAX], s_w[DEC_KMAX];
+    __shared__ int s_live[DEC_KMAX];   // IDS: slots whose ids lie in [0, E)
     __shared__ float s_hg[2 * DEC_PMAX];
     __shared__ float s_z[DEC_KMAX * DEC_CMAX];
-    __shared__ int s_list[DEC_MAX_GRID];   // units still missing after a poll
+    __shared__ __attribute__((aligned(16))) int s_list[DEC_MAX_GRID];   // units still missing after a poll (IDS: x's Q8_K before)
     __shared__ int s_fail, s_nmiss, s_wmiss[DEC_WAVES];
     __shared__ double s_red[NORM_T], s_nsum;   // norm of x
 
@@ -537,100 +570,115 @@ __global__ void __launch_bounds__(DEC_THREADS) k_decode1(DecArgs g) {
     const bool do_c = n0 < D;
     const float resv = (do_c && tid < C && g.res) ? g.res[n0 + tid] : 0.f;
 
-    // ---- A: router row wg (wave 0) and Q8_K of x block wg (wave 1); the
-    // logit is published only once this WG's Q8_K of x is out.  With a norm of
-    // x, every WG first normalizes x into LDS (s_dn: phase B parks down rows
-    // there later) while wave 0's row loads stream.
-    float4_t wrow[16];
-    if (wave == 0 && wg < E) dec_row_issue(g, wg, lane, wrow);
-    const float4_t *sxn = nullptr;
-    if (g.norm.kind != NORM_NONE) {
-        dec_norm_stage(g, (float4_t *)&s_dn[0][0], s_red, &s_nsum);
-        sxn = (const float4_t *)&s_dn[0][0];
-    }
-    float logit = 0.f;
-    if (wave == 0 && wg < E) logit = dec_row_finish(g, wg, lane, wrow, sxn);
-    else if (wave == 1 && wg < NB) dec_q8k_x(g, wg, lane, sxn);
-    vm_drain();
-    dec_lds_barrier();
-    if (wave == 0 && lane == 0 && wg < E) tw_store(g.tw + DEC_TW_LOGIT + wg, tag, __builtin_bit_cast(uint32_t, logit));
-
-    // ---- every logit (and so every Q8_K block of x); an A unit still missing
-    // after g.rescue_polls tries is computed here and stored again (same bits):
-    // no WG waits on a WG that is not running
     unsigned spins = 0;
-    for (;;) {
-        bool have = true;
-        if (tid < E) {
-            uint32_t v;
-            have = tw_wait1(g.tw + DEC_TW_LOGIT + tid, tag, g.rescue_polls, v);
-            if (have) s_logit[tid] = as_float(v);
-        }
-        if (dec_none_missing(s_wmiss, !have)) break;
-        const int nmiss = dec_missing(&s_nmiss, s_list, tid, -1, !have, false);
-        spins += g.rescue_polls + 1;
-        if (spins > DEC_SPIN_LIMIT) {
-            ok = false;
-            break;
-        }
-        for (int m = wave; m < nmiss; m += DEC_WAVES) {
-            const int a = __builtin_amdgcn_readfirstlane(s_list[m]);
-            if (a < NB) dec_q8k_x(g, a, lane, sxn);
-            float4_t wr[16];
-            dec_row_issue(g, a, lane, wr);
-            const float lv = dec_row_finish(g, a, lane, wr, sxn);
-            vm_drain();   // the x block is out before the logit
-            if (lane == 0) tw_store(g.tw + DEC_TW_LOGIT + a, tag, __builtin_bit_cast(uint32_t, lv));
-        }
-    }
-
-    // ---- B: routing (every WG), DMA of its gate/up and down rows
-    if (tid < DEC_KMAX) s_sel[tid] = tid < K ? tid : 0;
-    dec_lds_barrier();
     // this lane's activation piece: row group of LPR = 8*NB lanes, block bq,
-    // piece sl (every logit is in, so the Q8_K of x is too)
+    // piece sl
     const int LPR = 8 * NB, RPS = 64 / LPR;
     const int rr = lane / LPR, bq = (lane % LPR) >> 3, sl = lane & 7;
-    const Q4X xg = dec_q4x_load(g.xq, g.xbs, g.xd, D, bq, sl);
-    {
-        // rank of expert e = #{i : l_i > l_e} + #{i < e : l_i == l_e}; the K
-        // lowest ranks in rank order are ggml_top_k's stable descending pick.
-        // 8, 4 or 2 lanes per expert (E <= 64, 128, 256), each comparing a
-        // share of the logits
-        const int tpe = E <= DEC_THREADS / 8 ? 8 : E <= DEC_THREADS / 4 ? 4 : 2;
-        const int e = tid / tpe, j = tid % tpe;
-        int cnt = 0;
-        float ve = 0.f;
-        if (e < E) {
-            ve = s_logit[e];
-#pragma unroll 8
-            for (int i = j; i < E; i += tpe) {
-                const float vi = s_logit[i];
-                cnt += (int)(vi > ve) | ((int)(vi == ve) & (int)(i < e));
+    Q4X xg;
+    float4_t xids = {0.f, 0.f, 0.f, 0.f};   // IDS: this wave's block of x, and slot tid's routing
+    int my_gu = 0, my_dn = 0;
+    float my_w = 0.f;
+    if constexpr (IDS) {
+        if (wave < NB) xids = *(const float4_t *)(g.x + wave * QK + 4 * lane);
+        if (tid < K) {
+            my_gu = g.ids_gu[tid];
+            my_dn = g.ids_dn[tid];
+            my_w = g.wts[tid];
+        }
+    } else {
+        // ---- A: router row wg (wave 0) and Q8_K of x block wg (wave 1); the
+        // logit is published only once this WG's Q8_K of x is out.  With a norm of
+        // x, every WG first normalizes x into LDS (s_dn: phase B parks down rows
+        // there later) while wave 0's row loads stream.
+        float4_t wrow[16];
+        if (wave == 0 && wg < E) dec_row_issue(g, wg, lane, wrow);
+        const float4_t *sxn = nullptr;
+        if (g.norm.kind != NORM_NONE) {
+            dec_norm_stage(g, (float4_t *)&s_dn[0][0], s_red, &s_nsum);
+            sxn = (const float4_t *)&s_dn[0][0];
+        }
+        float logit = 0.f;
+        if (wave == 0 && wg < E) logit = dec_row_finish(g, wg, lane, wrow, sxn);
+        else if (wave == 1 && wg < NB) dec_q8k_x(g, wg, lane, sxn);
+        vm_drain();
+        dec_lds_barrier();
+        if (wave == 0 && lane == 0 && wg < E) tw_store(g.tw + DEC_TW_LOGIT + wg, tag, __builtin_bit_cast(uint32_t, logit));
+
+        // ---- every logit (and so every Q8_K block of x); an A unit still missing
+        // after g.rescue_polls tries is computed here and stored again (same bits):
+        // no WG waits on a WG that is not running
+        for (;;) {
+            bool have = true;
+            if (tid < E) {
+                uint32_t v;
+                have = tw_wait1(g.tw + DEC_TW_LOGIT + tid, tag, g.rescue_polls, v);
+                if (have) s_logit[tid] = as_float(v);
+            }
+            if (dec_none_missing(s_wmiss, !have)) break;
+            const int nmiss = dec_missing(&s_nmiss, s_list, tid, -1, !have, false);
+            spins += g.rescue_polls + 1;
+            if (spins > DEC_SPIN_LIMIT) {
+                ok = false;
+                break;
+            }
+            for (int m = wave; m < nmiss; m += DEC_WAVES) {
+                const int a = __builtin_amdgcn_readfirstlane(s_list[m]);
+                if (a < NB) dec_q8k_x(g, a, lane, sxn);
+                float4_t wr[16];
+                dec_row_issue(g, a, lane, wr);
+                const float lv = dec_row_finish(g, a, lane, wr, sxn);
+                vm_drain();   // the x block is out before the logit
+                if (lane == 0) tw_store(g.tw + DEC_TW_LOGIT + a, tag, __builtin_bit_cast(uint32_t, lv));
             }
         }
-        cnt += dpp_i<0xB1>(cnt);
-        if (tpe >= 4) cnt += dpp_i<0x4E>(cnt);
-        if (tpe >= 8) cnt += dpp_i<0x141>(cnt);
-        if (e < E && j == 0 && cnt < K) {
-            s_sel[cnt] = e;
-            s_val[cnt] = ve;
-        }
-    }
-    dec_lds_barrier();
 
-    const int64_t pairs = (int64_t)K * I;
+        // ---- B: routing (every WG), DMA of its gate/up and down rows
+        if (tid < DEC_KMAX) s_sel[tid] = tid < K ? tid : 0;
+        dec_lds_barrier();
+        // (every logit is in, so the Q8_K of x is too)
+        xg = dec_q4x_load(g.xq, g.xbs, g.xd, D, bq, sl);
+        {
+            // rank of expert e = #{i : l_i > l_e} + #{i < e : l_i == l_e}; the K
+            // lowest ranks in rank order are ggml_top_k's stable descending pick.
+            // 8, 4 or 2 lanes per expert (E <= 64, 128, 256), each comparing a
+            // share of the logits
+            const int tpe = E <= DEC_THREADS / 8 ? 8 : E <= DEC_THREADS / 4 ? 4 : 2;
+            const int e = tid / tpe, j = tid % tpe;
+            int cnt = 0;
+            float ve = 0.f;
+            if (e < E) {
+                ve = s_logit[e];
+#pragma unroll 8
+                for (int i = j; i < E; i += tpe) {
+                    const float vi = s_logit[i];
+                    cnt += (int)(vi > ve) | ((int)(vi == ve) & (int)(i < e));
+                }
+            }
+            cnt += dpp_i<0xB1>(cnt);
+            if (tpe >= 4) cnt += dpp_i<0x4E>(cnt);
+            if (tpe >= 8) cnt += dpp_i<0x141>(cnt);
+            if (e < E && j == 0 && cnt < K) {
+                s_sel[cnt] = e;
+                s_val[cnt] = ve;
+            }
+        }
+        dec_lds_barrier();
+    }
+
+    // (32-bit: the unit arithmetic sits in front of the weight loads, and a
+    // 64-bit division is some 150 instructions)
+    const uint32_t pairs = (uint32_t)(K * I);
     const int P = g.P, R = P / 4;
-    const int UB = (int)(pairs / P);          // gate/up units of P (h, g) row pairs
-    const int64_t q0 = (int64_t)wg * P;
-    const bool do_b = q0 < pairs;
+    const int UB = (int)(pairs / (uint32_t)P);          // gate/up units of P (h, g) row pairs
+    const bool do_b = (uint32_t)(wg * P) < pairs;
     uint32_t dn_shift = 0;
     // DMA of unit u's gate/up rows into s_gu (wave v: rows v % 4 of the h
     // (v < 4) or g half)
     auto b_issue = [&](int u, bool on) {
-        const int64_t q = (int64_t)u * P;
-        const int kb = on ? (int)(q / I) : 0, ib = on ? (int)(q % I) : 0;
-        int eb = __builtin_amdgcn_readfirstlane(s_sel[kb]);
+        const uint32_t q = (uint32_t)(u * P);
+        const int kb = on ? (int)(q / (uint32_t)I) : 0, ib = on ? (int)(q % (uint32_t)I) : 0;
+        int eb = IDS ? g.ids_gu[kb] : __builtin_amdgcn_readfirstlane(s_sel[kb]);
         eb = eb < 0 ? 0 : (eb >= E ? E - 1 : eb);
         const bool hpart = wave < 4;
         const ExpertMat &m = (hpart || g.fused) ? g.gate : g.up;
@@ -679,9 +727,8 @@ __global__ void __launch_bounds__(DEC_THREADS) k_decode1(DecArgs g) {
     // then the unit's completion word once wave 0's stores are out (P <= 64:
     // every store comes from wave 0)
     auto b_publish = [&](int u, bool owner) {
-        const int64_t q = (int64_t)u * P;
         if (tid < P)
-            st_dev4(g.actf, 4u * (uint32_t)(q + tid), __builtin_bit_cast(uint32_t, act_pair(g.act, s_hg[tid], s_hg[P + tid])));
+            st_dev4(g.actf, 4u * (uint32_t)(u * P + tid), __builtin_bit_cast(uint32_t, act_pair(g.act, s_hg[tid], s_hg[P + tid])));
         if (wave == 0) {
             vm_drain();
             if (lane == 0) tw_store(g.tw + DEC_TW_BDONE + u, tag, 1u);
@@ -693,7 +740,7 @@ __global__ void __launch_bounds__(DEC_THREADS) k_decode1(DecArgs g) {
     u32x4 dnv[DEC_DN_SEG];
     {
         const int k = wave < K ? wave : 0;
-        int ed = __builtin_amdgcn_readfirstlane(s_sel[k]);
+        int ed = IDS ? g.ids_dn[k] : __builtin_amdgcn_readfirstlane(s_sel[k]);
         ed = ed < 0 ? 0 : (ed >= E ? E - 1 : ed);
         const DecChunk c = dec_chunk(g.down, ed, n0, C, do_c && wave < K);
         dn_shift = c.shift;
@@ -703,32 +750,45 @@ __global__ void __launch_bounds__(DEC_THREADS) k_decode1(DecArgs g) {
         for (int s = 0; s < DEC_DN_SEG; ++s) dnv[s] = __builtin_amdgcn_raw_buffer_load_b128(r, 1024 * s + 16 * lane, 0, 0);
     }
 
-    if (wave == 0) {
-        const float myval = lane < K ? s_val[lane] : 0.f;
-        const float myw = softmax_selected_wave(myval, K, lane);
-        if (lane < K) s_w[lane] = myw;
-        if (wg == 0 && lane < K) {
-            g.sel[lane] = s_sel[lane];
-            g.w[lane] = myw;
+    if constexpr (IDS) {
+        if (wave < NB) dec_q8k_x_lds(xids, (uint8_t *)s_list, wave, lane);
+        if (tid < K) {
+            const int bad_gu = (unsigned)my_gu >= (unsigned)E, bad_dn = (unsigned)my_dn >= (unsigned)E;
+            s_live[tid] = !(bad_gu | bad_dn);
+            s_w[tid] = my_w;
+            const int bad = bad_gu + (g.ids_dn != g.ids_gu ? bad_dn : 0);
+            if (wg == 0 && bad) atomicAdd(g.bad_total, bad);
         }
-    }
-    if (wg == 0) {
-        if (tid < E) g.logits[tid] = s_logit[tid];
-        // single-token dispatch: one list entry per selected expert
-        for (int e = tid; e < E; e += DEC_THREADS) {
-            int cnt = 0, below = 0, slot = 0;
-            for (int k = 0; k < K; ++k) {
-                if (s_sel[k] == e) {
-                    cnt++;
-                    slot = k;
-                }
-                below += s_sel[k] < e;
+        dec_lds_barrier();
+        xg = dec_q4x_lds((const uint8_t *)s_list, bq, sl);
+    } else {
+        if (wave == 0) {
+            const float myval = lane < K ? s_val[lane] : 0.f;
+            const float myw = softmax_selected_wave(myval, K, lane);
+            if (lane < K) s_w[lane] = myw;
+            if (wg == 0 && lane < K) {
+                g.sel[lane] = s_sel[lane];
+                g.w[lane] = myw;
             }
-            g.counts[e] = cnt;
-            g.offsets[e] = below;
-            if (cnt) g.perm[below] = slot;
         }
-        if (tid == 0) g.offsets[E] = K;
+        if (wg == 0) {
+            if (tid < E) g.logits[tid] = s_logit[tid];
+            // single-token dispatch: one list entry per selected expert
+            for (int e = tid; e < E; e += DEC_THREADS) {
+                int cnt = 0, below = 0, slot = 0;
+                for (int k = 0; k < K; ++k) {
+                    if (s_sel[k] == e) {
+                        cnt++;
+                        slot = k;
+                    }
+                    below += s_sel[k] < e;
+                }
+                g.counts[e] = cnt;
+                g.offsets[e] = below;
+                if (cnt) g.perm[below] = slot;
+            }
+            if (tid == 0) g.offsets[E] = K;
+        }
     }
 
     if (do_b) b_dots();
@@ -877,7 +937,8 @@ __global__ void __launch_bounds__(DEC_THREADS) k_decode1(DecArgs g) {
     const bool failed = s_fail != 0;
     if (do_c && tid < C) {
         double s = 0.0;
-        for (int k = 0; k < K; ++k) s = s + (double)(s_z[k * C + tid] * s_w[k]);
+        for (int k = 0; k < K; ++k)
+            if (!IDS || s_live[k]) s = s + (double)(s_z[k * C + tid] * s_w[k]);
         const float moe = (float)s;
         float v = g.res ? resv + moe : moe;
         if (failed) v = __builtin_nanf("");
@@ -1495,24 +1556,30 @@ int launch_decodeb(const DecArgs &g, int grid, hipStream_t st) {
     return hip_check_launch();
 }
 
-template <int DT>
+template <int DT, bool IDS>
 static const void *decode1_fn(int nbi) {
     switch (nbi) {
-    case 1: return (const void *)k_decode1<DT, 1>;
-    case 2: return (const void *)k_decode1<DT, 2>;
-    case 3: return (const void *)k_decode1<DT, 3>;
-    case 4: return (const void *)k_decode1<DT, 4>;
-    case 5: return (const void *)k_decode1<DT, 5>;
-    case 6: return (const void *)k_decode1<DT, 6>;
-    case 7: return (const void *)k_decode1<DT, 7>;
-    case 8: return (const void *)k_decode1<DT, 8>;
+    case 1: return (const void *)k_decode1<DT, 1, IDS>;
+    case 2: return (const void *)k_decode1<DT, 2, IDS>;
+    case 3: return (const void *)k_decode1<DT, 3, IDS>;
+    case 4: return (const void *)k_decode1<DT, 4, IDS>;
+    case 5: return (const void *)k_decode1<DT, 5, IDS>;
+    case 6: return (const void *)k_decode1<DT, 6, IDS>;
+    case 7: return (const void *)k_decode1<DT, 7, IDS>;
+    case 8: return (const void *)k_decode1<DT, 8, IDS>;
     default: return nullptr;
     }
+}
+static const void *decode1_fn(int dt, bool ids, int nbi) {
+    if (dt == 12) return ids ? decode1_fn<12, true>(nbi) : decode1_fn<12, false>(nbi);
+    if (dt == 14) return ids ? decode1_fn<14, true>(nbi) : decode1_fn<14, false>(nbi);
+    return nullptr;
 }
 
 int launch_decode1(const DecArgs &g, int grid, hipStream_t st) {
     const int nbi = g.I / QK;
-    const void *fn = g.down.type == 12 ? decode1_fn<12>(nbi) : g.down.type == 14 ? decode1_fn<14>(nbi) : nullptr;
+    if (g.ids_gu && (!g.ids_dn || !g.wts || !g.bad_total || g.norm.kind != NORM_NONE || g.D > 8 * QK)) return -6;
+    const void *fn = decode1_fn(g.down.type, g.ids_gu != nullptr, nbi);
     if (!fn) return -3;
     void *args[] = {(void *)&g};
     const hipError_t e = hipLaunchKernel(fn, dim3(grid), dim3(DEC_THREADS), args, 0, st);
@@ -1528,8 +1595,7 @@ int decode1_max_grid(int device, int *grid) {
     for (int dt = 12; dt <= 14; dt += 2)
         for (int nbi = 1; nbi <= 8; ++nbi) {
             int p = 0;
-            e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&p, dt == 12 ? decode1_fn<12>(nbi) : decode1_fn<14>(nbi),
-                                                             DEC_THREADS, 0);
+            e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&p, decode1_fn(dt, false, nbi), DEC_THREADS, 0);
             if (e != hipSuccess) return record_hip_error(e);
             per = imin(per, p);
         }

@@ -331,6 +331,13 @@ struct DecArgs {
     unsigned *err;                // set when a wait gave up (output is NaN)
     unsigned rescue_polls;        // polls for another WG's unit before computing it here
     NormParams norm;              // k_decode1: the norm of x applied in the kernel (kind NORM_NONE: x as given)
+    // k_decode1, the caller's routing (else NULL): expert ids [K] of the gate/up
+    // and down products and weights [K] in place of the router's; ids outside
+    // [0, E) leave their slot out and are counted in bad_total; no routing
+    // outputs, no norm, x and out disjoint
+    const int32_t *ids_gu, *ids_dn;
+    const float *wts;
+    int32_t *bad_total;
 };
 constexpr int DEC_MAX_GRID = 1024;
 // epoch-tagged words: the E router logits, then one per gate/up unit

@@ -558,24 +558,41 @@ int gb_bm(const mi_moe_ctx *c, int64_t rows, int E, int64_t ncols) {
 // token (larger calls run in passes)
 int64_t gb_max_tokens(int64_t halfs) { return GB_MAX_X / (2 * halfs); }
 bool gb_strides_ok(const mi_tensor &t) { return (int64_t)t.nb[1] <= GB_MAX_ROW_BYTES; }
+// the grouped GEMM for a routed call (row strides past its 32-bit offsets keep the GEMV)
+bool gb_path(const mi_moe_ctx *c, const mi_moe_layer *L, int64_t T) {
+    return use_gemm_wide(c, T, L->n_expert_used, L->n_expert) && gb_strides_ok(L->gate) && gb_strides_ok(L->down) &&
+           (!act_gated(L->act) || L->fused_gate_up || gb_strides_ok(L->up));
+}
+// The shared expert in the routed experts' own GEMM launches: the same table
+// types and activation (one kernel), one pass.  By itself it is a chain of six
+// launches (ids, dispatch, operand, two products of a few work-groups each,
+// combine): nemotronomni T = 200 394 us with the chain (90 us of it), 331
+// with its work-groups in the two routed launches (134 + 127 -> 166 + 160 us).
+bool gb_shared_ok(const mi_moe_ctx *c, const mi_moe_layer *L, int64_t T) {
+    if (!is_b32f(L->gate.type) || !gb_path(c, L, T)) return false;
+    if (L->sh_gate.type != L->gate.type || L->sh_down.type != L->down.type || L->sh_act != L->act) return false;
+    if (!gb_strides_ok(L->sh_gate) || !gb_strides_ok(L->sh_down) || (act_gated(L->act) && !gb_strides_ok(L->sh_up)))
+        return false;
+    const int64_t K = L->n_expert_used;
+    return T <= gb_max_tokens(std::max({round_up(L->n_embd, 64), K * round_up(L->n_ff, 64), round_up(L->sh_n_ff, 64)}));
+}
 
 // routed FFN body of a layer with Q4_0 / Q5_0 / Q8_0 / F16 tables: the rows
 // converted to each product's ggml vec_dot_type (Q8_0 or fp16), fp32 slot
 // rows into the combine.  Below the GEMM threshold the grouped GEMV
 // (k_b32.hip), GLU rows in fp32; above it the grouped MFMA GEMM (k_gb.hip),
 // whose gate/up launch writes the down product's operand rows itself.
-// Arguments as run_experts.
+// Arguments as run_experts; sh_here: the shared expert too (gb_shared_ok),
+// its rows' weights in sh_w (NULL: 1), added to the routed sum.
 int run_experts_b32(mi_moe_ctx *c, const mi_moe_layer *L, const float *x, int64_t T, const int32_t *ids_gu,
                     const int32_t *ids_dn, const float *w, const float *res, float *out, hipStream_t st,
-                    bool check_ids, const float *add) {
+                    bool check_ids, const float *add, bool sh_here = false, const float *sh_w = nullptr) {
     const int D = L->n_embd, E = L->n_expert, K = L->n_expert_used, I = L->n_ff;
     const int64_t rows = T * K;
     const int max_active = (int)std::min<int64_t>(E, rows);
     const bool same_ids = ids_gu == ids_dn;
     const bool gated = act_gated(L->act);
-    // (row strides past the GEMM's 32-bit offsets keep the GEMV)
-    const bool gemm = use_gemm_wide(c, T, K, E) && gb_strides_ok(L->gate) && gb_strides_ok(L->down) &&
-                      (!gated || L->fused_gate_up || gb_strides_ok(L->up));
+    const bool gemm = gb_path(c, L, T);
     const int64_t ldx = round_up(D, 64), ldi = round_up(I, 64);
     const int64_t tmax = gb_max_tokens(std::max(ldx, K * ldi));
     if (gemm && T > tmax) {
@@ -617,6 +634,15 @@ int run_experts_b32(mi_moe_ctx *c, const mi_moe_layer *L, const float *x, int64_
         a.perm = dg.perm; a.tile_e = dg.tile_e; a.tile_start = dg.tile_start; a.tile_rows = dg.tile_rows;
         a.n_tiles = dg.n_tiles; a.max_tiles = max_tiles; a.bm = bm;
         a.ncols = I; a.xo = c->aact.h; a.ldo = ldi; a.next_f16 = L->down.type == MI_TYPE_F16;
+        if (sh_here) {
+            a.sh_rows = T;
+            a.sh.a = as_mat(L->sh_gate);
+            if (gated) a.sh.b = as_mat(L->sh_up);
+            a.sh.I = a.sh.ncols = L->sh_n_ff;
+            a.sh.xh = a.xh; a.sh.ldx = a.ldx; a.sh.xrows = T;
+            // (f1 is free on this path, and holds 2 cap_I floats per slot)
+            a.sh.xo = (_Float16 *)c->f1; a.sh.ldo = round_up(L->sh_n_ff, 64);
+        }
         TRY(launch_gb(a, st));
         stage_end(c, "gate_up", st);
         GBArgs d = {};
@@ -625,6 +651,14 @@ int run_experts_b32(mi_moe_ctx *c, const mi_moe_layer *L, const float *x, int64_
         d.perm = dd.perm; d.tile_e = dd.tile_e; d.tile_start = dd.tile_start; d.tile_rows = dd.tile_rows;
         d.n_tiles = dd.n_tiles; d.max_tiles = max_tiles; d.bm = bm;
         d.y = c->z; d.ldy = D; d.ncols = D;
+        if (sh_here) {
+            d.sh_rows = T;
+            d.sh.a = as_mat(L->sh_down);
+            d.sh.xh = a.sh.xo; d.sh.ldx = a.sh.ldo; d.sh.xrows = T;
+            d.sh.y = c->sh_out; d.sh.ldy = d.sh.ncols = D;
+            d.sh_w = sh_w;
+            add = c->sh_out;
+        }
         TRY(launch_gb(d, st));
     } else {
         auto args_for = [&](const ExpertMat &a, const DispBuf &d, const ActBuf &ab, int ne11) {
@@ -661,12 +695,14 @@ int run_experts_b32(mi_moe_ctx *c, const mi_moe_layer *L, const float *x, int64_
 // routed FFN body: ids (device [T][K]; gate/up and down may differ) and
 // weights w [T][K]; x_done: x is already in the x_q8_spec form; check_ids:
 // the ids come from the caller (dead slots are left out of the combine);
-// add: [T][D] added to the routed sum before the residual (or null)
+// add: [T][D] added to the routed sum before the residual (or null);
+// sh_here, sh_w: the shared expert in these launches (run_experts_b32)
 int run_experts(mi_moe_ctx *c, const mi_moe_layer *L, const float *x, int64_t T, const int32_t *ids_gu,
                 const int32_t *ids_dn, const float *w, const float *res, float *out, hipStream_t st,
                 bool x_done = false, bool check_ids = false, const float *add = nullptr,
-                bool disp_out = true) {
-    if (is_b32f(L->gate.type)) return run_experts_b32(c, L, x, T, ids_gu, ids_dn, w, res, out, st, check_ids, add);
+                bool disp_out = true, bool sh_here = false, const float *sh_w = nullptr) {
+    if (is_b32f(L->gate.type))
+        return run_experts_b32(c, L, x, T, ids_gu, ids_dn, w, res, out, st, check_ids, add, sh_here, sh_w);
     const int D = L->n_embd, E = L->n_expert, K = L->n_expert_used, I = L->n_ff;
     const int64_t rows = T * K;
     const int max_active = (int)std::min<int64_t>(E, rows);
@@ -862,9 +898,19 @@ int run_experts(mi_moe_ctx *c, const mi_moe_layer *L, const float *x, int64_t T,
     return MI_MOE_OK;
 }
 
+// The shared expert's ids (all 0) and weights: 1, or the sigmoid of the scalar
+// gate row (a one-expert router in the router's fixed fp64 order).
+int shared_weights(mi_moe_ctx *c, const mi_moe_layer *L, const float *x, int64_t T, hipStream_t st) {
+    const float *lg = nullptr;
+    if (L->sh_gate_inp) {
+        TRY(launch_front(L->sh_gate_inp, nullptr, x, L->n_embd, T, L->n_embd, 1, c->sh_logit, nullptr, st));
+        lg = c->sh_logit;
+    }
+    return launch_shared_gate(lg, T, c->sh_ids, c->sh_w, st);
+}
+
 // The shared expert of every token into c->sh_out: a one-expert layer whose
-// tokens all select expert 0 with weight 1 or the sigmoid of the scalar gate
-// row (a one-expert router in the router's fixed fp64 order).
+// tokens all select expert 0.
 int run_shared(mi_moe_ctx *c, const mi_moe_layer *L, const float *x, int64_t T, hipStream_t st) {
     mi_moe_layer S = {};
     S.n_embd = L->n_embd;
@@ -876,12 +922,7 @@ int run_shared(mi_moe_ctx *c, const mi_moe_layer *L, const float *x, int64_t T, 
     S.down = L->sh_down;
     S.fused_gate_up = 0;
     S.act = L->sh_act;
-    const float *lg = nullptr;
-    if (L->sh_gate_inp) {
-        TRY(launch_front(L->sh_gate_inp, nullptr, x, L->n_embd, T, L->n_embd, 1, c->sh_logit, nullptr, st));
-        lg = c->sh_logit;
-    }
-    TRY(launch_shared_gate(lg, T, c->sh_ids, c->sh_w, st));
+    TRY(shared_weights(c, L, x, T, st));
     TRY(run_experts(c, &S, x, T, c->sh_ids, c->sh_ids, c->sh_w, nullptr, c->sh_out, st));
     stage_end(c, "shared_expert", st);
     return MI_MOE_OK;
@@ -1223,9 +1264,13 @@ int forward_impl(mi_moe_ctx *c, const mi_moe_layer *L, const float *x, int64_t T
         stage_end(c, "norm", st);
         x = c->xn;
     }
-    // the shared expert first (its own Q8_K of x; the routed block's follows)
+    // the shared expert first (its own Q8_K of x; the routed block's follows),
+    // unless it rides in the routed launches
     const float *add = nullptr;
-    if (L->sh_n_ff > 0) {
+    const bool sh_here = L->sh_n_ff > 0 && gb_shared_ok(c, L, T);
+    if (sh_here) {
+        if (L->sh_gate_inp) TRY(shared_weights(c, L, x, T, st));
+    } else if (L->sh_n_ff > 0) {
         TRY(run_shared(c, L, x, T, st));
         add = c->sh_out;
     }
@@ -1262,7 +1307,8 @@ int forward_impl(mi_moe_ctx *c, const mi_moe_layer *L, const float *x, int64_t T
         }
         stage_end(c, "topk_softmax", st);
         TRY(run_experts(c, L, x, T, c->sel, c->sel, c->w, res, out, st, x_done, false, add,
-                        routing && (routing->counts || routing->offsets || routing->perm)));
+                        routing && (routing->counts || routing->offsets || routing->perm), sh_here,
+                        L->sh_gate_inp ? c->sh_w : nullptr));
     }
     if (routing) {
         const DispBuf &d = c->disp[0];
@@ -1409,8 +1455,8 @@ int mi_moe_expert_ffn(mi_moe_ctx *c, const mi_moe_layer *L, const float *x, int6
     hipStream_t st = (hipStream_t)stream;
     stage_begin(c, st);
     // One or two tokens on the fused kernel, a launch each (layer us against
-    // the chain: qwen3omni 16.2 / 29.4 at one, 32.8 / 35.5 at two, three
-    // tokens 48.7 / 45.7; moondream3 18.5 / 33 and 37 / 42), unless the caller
+    // the chain: qwen3omni 16.2 / 29.4 at one, 32.2 / 35.5 at two, the chain at
+    // three 45.6; moondream3 36.5 / 42.0 at two), unless the caller
     // asked for the GEMM at that size or out overlaps what every work-group of
     // the kernel reads (a late one may read after others wrote their columns).
     int P = 0, C = 0;

@@ -330,7 +330,7 @@ __device__ __forceinline__ void gb_kloop(rsrc_t rx, const uint32_t *aoff, const 
 // LDS (its weight buffer) into rows, four lanes per row; the arithmetic and
 // bits of launch_prep_b32 on the fp32 values.
 template <typename V>
-__device__ __forceinline__ void gb_next_rows(const GBArgs &g, float *lds, int rt, int mrows, int64_t n, int lane,
+__device__ __forceinline__ void gb_next_rows(const GBSide &g, int next_f16, float *lds, int rt, int mrows, int64_t n, int lane,
                                              const int *s_p, V &&v) {
     const int l32 = lane & 31, h = lane >> 5;
 #pragma unroll
@@ -341,25 +341,27 @@ __device__ __forceinline__ void gb_next_rows(const GBArgs &g, float *lds, int rt
         const float4_t a = *(const float4_t *)(lds + 8 * lane), b = *(const float4_t *)(lds + 8 * lane + 4);
         wave_lds_sync();   // (rewritten next)
         const float x[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
-        const uint4 o = g.next_f16 ? b32_f16x8(x) : b32_q8x8(x);
+        const uint4 o = next_f16 ? b32_f16x8(x) : b32_q8x8(x);
         const int m = 32 * rt + 16 * half + (lane >> 2);
         if (m < mrows) *(uint4 *)(g.xo + (int64_t)s_p[m] * g.ldo + n + 8 * (lane & 3)) = o;
     }
 }
 
 template <int ACT, int NA>
-__device__ __forceinline__ void gb_glu_out(const GBArgs &g, const f32x16 (&acc)[NA][2], int nrt, int mrows, int64_t n0,
+__device__ __forceinline__ void gb_glu_out(const GBSide &g, int next_f16, const f32x16 (&acc)[NA][2], int nrt, int mrows, int64_t n0,
                                            int lane, const int *s_p, float *lds) {
     const bool in = n0 < g.ncols;   // (the padding columns of an odd block count: zeros)
 #pragma unroll
     for (int rt = 0; rt < NA; ++rt)
         if (rt < nrt)
-            gb_next_rows(g, lds, rt, mrows, n0, lane, s_p, [&](int i) __attribute__((always_inline)) {
+            gb_next_rows(g, next_f16, lds, rt, mrows, n0, lane, s_p, [&](int i) __attribute__((always_inline)) {
                 return in ? act_pair(ACT, acc[rt][0][i], acc[rt][1][i]) : 0.f;
             });
 }
 
-template <int WT, int EPI, int BM, int NW, int KG>
+// SH: the shared expert's rows are in this launch (GBArgs::sh; a form of its
+// own, the selection in front of the first loads costs 1 - 2 us per layer)
+template <int WT, int EPI, int BM, int NW, int KG, bool SH>
 __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) k_gb(GBArgs g) {
 #ifdef __HIP_DEVICE_COMPILE__   // (the host pass needs the stub alone, and rejects the builtins' second instantiation)
     constexpr int NA = BM / 32;
@@ -367,28 +369,45 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
     __shared__ __attribute__((aligned(128))) _Float16 As0[BM * 64 * (KG / 2)];
     __shared__ __attribute__((aligned(128))) _Float16 As1[BM * 64 * (KG / 2)];
     __shared__ __attribute__((aligned(128))) uint8_t Ws[NW * WREG];
-    // work-group 8 q + x on XCD x: the x-th eighth of the tiles in expert
-    // order, one after another, column tile q % nct (the column tiles of one
-    // row tile share that XCD's L2 for the activations, the row tiles of one
-    // expert for the weights)
-    const int lin = blockIdx.x, qq = lin >> 3, nt = *g.n_tiles, per = (nt + 7) >> 3;
-    const int kk = qq / g.nct, ctile = qq - kk * g.nct, tile = (lin & 7) * per + kk;
-    if (kk >= per || tile >= nt) return;
-    const int e = g.tile_e[tile], start = g.tile_start[tile], mrows = g.tile_rows[tile];
+    // The shared expert's work-groups first: on XCD x the column tiles c % 8
+    // = x, the row tiles of each one after another (its weights from that
+    // XCD's L2).  Then work-group 8 q + x on XCD x: the x-th eighth of the
+    // tiles in expert order, one after another, column tile q % nct (the
+    // column tiles of one row tile share that XCD's L2 for the activations,
+    // the row tiles of one expert for the weights).
+    const bool shared = SH && (int)blockIdx.x < g.sh_wgs;
+    const GBSide s = shared ? g.sh : (const GBSide &)g;
+    int e = 0, start, mrows, ctile;
+    if (shared) {
+        const int qq = blockIdx.x >> 3, cq = qq / g.sh_tiles;
+        ctile = 8 * cq + ((int)blockIdx.x & 7);
+        if (ctile >= s.nct) return;
+        start = BM * (qq - cq * g.sh_tiles);
+        mrows = (int)g.sh_rows - start;
+        if (mrows > BM) mrows = BM;
+    } else {
+        const int lin = blockIdx.x - (SH ? g.sh_wgs : 0), qq = lin >> 3, nt = *g.n_tiles, per = (nt + 7) >> 3;
+        const int kk = qq / s.nct, tile = (lin & 7) * per + kk;
+        ctile = qq - kk * s.nct;
+        if (kk >= per || tile >= nt) return;
+        e = g.tile_e[tile];
+        start = g.tile_start[tile];
+        mrows = g.tile_rows[tile];
+    }
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nrt = (mrows + 31) >> 5;
     constexpr bool GLU = EPI == GB_GLU;
-    const int64_t K = g.a.K;
+    const int64_t K = s.a.K;
     const int64_t n0 = (int64_t)ctile * (GLU ? 32 * NW : 64 * NW) + (GLU ? 32 : 64) * wave;
-    const uint8_t *ma = g.a.data + (int64_t)e * g.a.mat_bytes;
+    const uint8_t *ma = s.a.data + (int64_t)e * s.a.mat_bytes;
     const int wbase = wave * WREG;
     const uint32_t b0 = (uint32_t)wbase, b1 = b0 + (uint32_t)WTILE;
     GBW<WT, KG> wd[2];
-    wd[0] = gb_wdesc<WT, KG>(ma, n0, g.a.N, g.a.row_bytes, K, lane, b0);
-    if (!GLU) wd[1] = gb_wdesc<WT, KG>(ma, n0 + 32, g.a.N, g.a.row_bytes, K, lane, b1);
-    else if (g.fused) wd[1] = gb_wdesc<WT, KG>(ma, g.I + n0, g.a.N, g.a.row_bytes, K, lane, b1);
-    else wd[1] = gb_wdesc<WT, KG>(g.b.data + (int64_t)e * g.b.mat_bytes, n0, g.b.N, g.b.row_bytes, K, lane, b1);
+    wd[0] = gb_wdesc<WT, KG>(ma, n0, s.a.N, s.a.row_bytes, K, lane, b0);
+    if (!GLU) wd[1] = gb_wdesc<WT, KG>(ma, n0 + 32, s.a.N, s.a.row_bytes, K, lane, b1);
+    else if (s.fused) wd[1] = gb_wdesc<WT, KG>(ma, s.I + n0, s.a.N, s.a.row_bytes, K, lane, b1);
+    else wd[1] = gb_wdesc<WT, KG>(s.b.data + (int64_t)e * s.b.mat_bytes, n0, s.b.N, s.b.row_bytes, K, lane, b1);
     // the tile's rows: the slot indices first (their loads ahead of the
     // weights', which stay in flight), as activation offsets of this lane's
     // loads and, for the epilogue, one per thread
@@ -398,9 +417,9 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
 #pragma unroll
     for (int j = 0; j < NAL; ++j) {
         const int r = 8 * (wave + NW * j) + (lane >> 3);
-        prow[j] = r < mrows ? g.perm[start + r] : -1;
+        prow[j] = r < mrows ? (shared ? start + r : g.perm[start + r]) : -1;
     }
-    const int my_p = tid < mrows ? g.perm[start + tid] : -1;
+    const int my_p = tid < mrows ? (shared ? start + tid : g.perm[start + tid]) : -1;
     asm volatile("" ::: "memory");   // (keeps the order)
 #pragma unroll
     for (int ct = 0; ct < 2; ++ct) wd[ct].issue(Ws + (wbase + ct * WTILE), 0);
@@ -408,9 +427,9 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
 #pragma unroll
     for (int j = 0; j < NAL; ++j)
         aoff[j] = prow[j] < 0 ? GB_FAR
-                              : (uint32_t)(g.ne11 == 1 ? prow[j] / g.K : prow[j]) * (2u * (uint32_t)g.ldx) +
+                              : (uint32_t)(g.ne11 == 1 && !shared ? prow[j] / g.K : prow[j]) * (2u * (uint32_t)s.ldx) +
                                     16u * (uint32_t)((lane & 7) ^ (lane >> 3));
-    const rsrc_t rx = gb_rsrc(g.xh, g.xbytes);
+    const rsrc_t rx = gb_rsrc(s.xh, s.xbytes);
     f32x16 acc[NA][2];
 #define GB_LOOP(N) gb_kloop<WT, N, NA, NW, BM, KG>(rx, aoff, wd, K, wave, lane, wbase, As0, As1, Ws, acc)
     if constexpr (NA == 1) GB_LOOP(1);
@@ -429,13 +448,13 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
     lds_barrier();
     const int l32 = lane & 31, h = lane >> 5;
     if constexpr (EPI == GB_GLU) {
-        if (n0 >= g.ldo) return;
+        if (n0 >= s.ldo) return;
         float *lds = (float *)(Ws + wbase);   // (no load is in flight and no other wave reads it)
         switch (g.act) {
-        case 0: gb_glu_out<0, NA>(g, acc, nrt, mrows, n0, lane, s_p, lds); break;
-        case 1: gb_glu_out<1, NA>(g, acc, nrt, mrows, n0, lane, s_p, lds); break;
-        case 2: gb_glu_out<2, NA>(g, acc, nrt, mrows, n0, lane, s_p, lds); break;
-        default: gb_glu_out<3, NA>(g, acc, nrt, mrows, n0, lane, s_p, lds); break;
+        case 0: gb_glu_out<0, NA>(s, g.next_f16, acc, nrt, mrows, n0, lane, s_p, lds); break;
+        case 1: gb_glu_out<1, NA>(s, g.next_f16, acc, nrt, mrows, n0, lane, s_p, lds); break;
+        case 2: gb_glu_out<2, NA>(s, g.next_f16, acc, nrt, mrows, n0, lane, s_p, lds); break;
+        default: gb_glu_out<3, NA>(s, g.next_f16, acc, nrt, mrows, n0, lane, s_p, lds); break;
         }
     } else {
 #pragma unroll
@@ -445,15 +464,18 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
             for (int rt = 0; rt < NA; ++rt) {
                 if (rt >= nrt) continue;
                 if constexpr (EPI == GB_RELU_SQR) {
-                    if (n < g.ldo)
-                        gb_next_rows(g, (float *)(Ws + wbase), rt, mrows, n, lane, s_p, [&](int i) __attribute__((always_inline)) {
-                            return n < g.ncols ? relu_sqr(acc[rt][ct][i]) : 0.f;
+                    if (n < s.ldo)
+                        gb_next_rows(s, g.next_f16, (float *)(Ws + wbase), rt, mrows, n, lane, s_p, [&](int i) __attribute__((always_inline)) {
+                            return n < s.ncols ? relu_sqr(acc[rt][ct][i]) : 0.f;
                         });
                 } else {
 #pragma unroll
                     for (int i = 0; i < 16; ++i) {
                         const int m = 32 * rt + 8 * (i >> 2) + 4 * h + (i & 3);
-                        if (m < mrows && n + l32 < g.ncols) g.y[(int64_t)s_p[m] * g.ldy + n + l32] = acc[rt][ct][i];
+                        if (m < mrows && n + l32 < s.ncols) {
+                            const float v = acc[rt][ct][i];
+                            s.y[(int64_t)s_p[m] * s.ldy + n + l32] = shared && g.sh_w ? v * g.sh_w[s_p[m]] : v;
+                        }
                     }
                 }
             }
@@ -475,25 +497,47 @@ static int gb_launch(const GBArgs &a, hipStream_t st) {
     constexpr int NS = WT == 1 ? 4 : 2, KS = WT == 1 || WT == 8 ? 2 : 4;
     const int nw = g.bm == GB_BM_LARGE ? 4 : NS;
     const int per = EPI == GB_GLU ? 32 * nw : 64 * nw;
-    const int64_t cols = EPI == GB_STORE ? g.ncols : g.ldo;   // (with the padding columns)
-    g.nct = (int)((cols + per - 1) / per);
-    const int64_t wgs = 8 * (int64_t)g.nct * ((g.max_tiles + 7) / 8);
+    auto column_tiles = [&](const GBSide &s) {   // (with the padding columns)
+        return (int)(((EPI == GB_STORE ? s.ncols : s.ldo) + per - 1) / per);
+    };
+    g.nct = column_tiles(g);
+    int64_t wgs = 8 * (int64_t)g.nct * ((g.max_tiles + 7) / 8);
+    g.sh_wgs = g.sh_tiles = 0;
+    if (g.sh_rows > 0) {
+        g.sh.nct = column_tiles(g.sh);
+        g.sh_tiles = (int)((g.sh_rows + g.bm - 1) / g.bm);
+        const int64_t sw = 8 * (int64_t)((g.sh.nct + 7) / 8) * g.sh_tiles;
+        if (sw > 0x7fffffff) return -6;
+        g.sh_wgs = (int)sw;
+        wgs += sw;
+    }
     if (wgs > 0x7fffffff) return -6;
     const dim3 grid((unsigned)wgs), block((unsigned)(64 * nw));
-    if (g.bm == GB_BM_LARGE) hipLaunchKernelGGL((k_gb<WT, EPI, GB_BM_LARGE, 4, 2>), grid, block, 0, st, g);
-    else hipLaunchKernelGGL((k_gb<WT, EPI, GB_BM_SMALL, NS, KS>), grid, block, 0, st, g);
+    if (g.sh_wgs) {
+        if (g.bm == GB_BM_LARGE) hipLaunchKernelGGL((k_gb<WT, EPI, GB_BM_LARGE, 4, 2, true>), grid, block, 0, st, g);
+        else hipLaunchKernelGGL((k_gb<WT, EPI, GB_BM_SMALL, NS, KS, true>), grid, block, 0, st, g);
+    } else {
+        if (g.bm == GB_BM_LARGE) hipLaunchKernelGGL((k_gb<WT, EPI, GB_BM_LARGE, 4, 2, false>), grid, block, 0, st, g);
+        else hipLaunchKernelGGL((k_gb<WT, EPI, GB_BM_SMALL, NS, KS, false>), grid, block, 0, st, g);
+    }
     return hip_check_launch();
+}
+
+static bool gb_side_ok(const GBArgs &g, const GBSide &s) {
+    if (s.a.K % 32 || s.ldx % 64 || (uintptr_t)s.xh % 16) return false;
+    if (s.xrows <= 0 || s.xrows * s.ldx * 2 > GB_MAX_X) return false;
+    if (s.a.row_bytes > GB_MAX_ROW_BYTES || (g.glu && !s.fused && s.b.row_bytes > GB_MAX_ROW_BYTES)) return false;
+    return !((g.glu || g.relu_sqr) && (s.ncols % 32 || s.ldo % 64 || !s.xo));
 }
 
 int launch_gb(const GBArgs &g, hipStream_t st) {
     if (g.max_tiles <= 0) return 0;
-    if (g.a.K % 32 || g.ldx % 64 || (uintptr_t)g.xh % 16) return -6;
     if (g.bm != GB_BM_SMALL && g.bm != GB_BM_LARGE) return -6;
-    if (g.xrows <= 0 || g.xrows * g.ldx * 2 > GB_MAX_X) return -6;
-    if (g.a.row_bytes > GB_MAX_ROW_BYTES || (g.glu && !g.fused && g.b.row_bytes > GB_MAX_ROW_BYTES)) return -6;
-    if ((g.glu || g.relu_sqr) && (g.ncols % 32 || g.ldo % 64 || !g.xo)) return -6;
+    if (!gb_side_ok(g, g)) return -6;
+    if (g.sh_rows > 0 && (!gb_side_ok(g, g.sh) || g.sh.a.type != g.a.type || g.sh_rows > g.sh.xrows)) return -6;
     GBArgs a = g;
     a.xbytes = (uint32_t)(g.xrows * g.ldx * 2);
+    a.sh.xbytes = (uint32_t)(g.sh.xrows * g.sh.ldx * 2);
 #define GB_TYPE(T)                                              \
     case T:                                                     \
         if (g.glu) return gb_launch<T, GB_GLU>(a, st);          \

@@ -284,22 +284,35 @@ int launch_gemv_b32(const B32Args &g, hipStream_t st);
 // activation rows leave as the next product's operand xo [p][ldo] (ldo =
 // ncols rounded up to 64, zeros past ncols; ncols % 32 == 0): fp16(v), or
 // their Q8_0 as fp16(d q), the bits of launch_prep_b32 on the fp32 values.
-struct GBArgs {
+//
+// A shared expert (sh_rows > 0) rides in the same launch: sh_rows rows (its
+// xh rows in order, no dispatch) through the tables and operands of sh, of
+// the same types, epilogue and act; sh_w: weights of its rows (plain product;
+// NULL: 1).
+struct GBSide {
     ExpertMat a, b;            // b: up table (separate gate/up GLU), else unused
-    int glu, fused, act;
-    int relu_sqr;              // one product, relu(v)^2 of it
+    int fused;
     int64_t I;
     const _Float16 *xh;
     int64_t ldx, xrows;
-    uint32_t xbytes;           // (set by launch_gb)
-    int ne11, K;
-    const int32_t *perm, *tile_e, *tile_start, *tile_rows, *n_tiles;
-    int max_tiles, bm, nct;    // nct: column tiles (set by launch_gb)
     float *y;
     int64_t ldy, ncols;
     _Float16 *xo;
     int64_t ldo;
+    uint32_t xbytes;           // (set by launch_gb)
+    int nct;                   // column tiles (set by launch_gb)
+};
+struct GBArgs : GBSide {
+    int glu, act;
+    int relu_sqr;              // one product, relu(v)^2 of it
+    int ne11, K;
+    const int32_t *perm, *tile_e, *tile_start, *tile_rows, *n_tiles;
+    int max_tiles, bm;
     int next_f16;
+    GBSide sh;
+    int64_t sh_rows;
+    const float *sh_w;
+    int sh_wgs, sh_tiles;      // (set by launch_gb)
 };
 constexpr int GB_BM_SMALL = 32, GB_BM_LARGE = 128;
 constexpr int64_t GB_MAX_X = 0xF0000000ll;          // bytes of xh (32-bit buffer offsets)

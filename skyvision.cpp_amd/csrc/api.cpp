@@ -563,14 +563,20 @@ bool gb_path(const mi_moe_ctx *c, const mi_moe_layer *L, int64_t T) {
     return use_gemm_wide(c, T, L->n_expert_used, L->n_expert) && gb_strides_ok(L->gate) && gb_strides_ok(L->down) &&
            (!act_gated(L->act) || L->fused_gate_up || gb_strides_ok(L->up));
 }
-// The shared expert in the routed experts' own GEMM launches: the same table
+// The GEMV runs the shared expert's tokens four to a pass over its rows, one
+// pass after another, beside the routed experts' work-groups: up to this many
+// (nemotronomni Q5_0 T = 1 / 4 / 16 with the chain 109 / 177 / 302 us, in the
+// launches 47 / 80 / 176, the faster GEMV included).
+constexpr int64_t GV_SHARED_T = 32;
+// The shared expert in the routed experts' own launches: the same table
 // types and activation (one kernel), one pass.  By itself it is a chain of six
 // launches (ids, dispatch, operand, two products of a few work-groups each,
 // combine): nemotronomni T = 200 394 us with the chain (90 us of it), 331
 // with its work-groups in the two routed launches (134 + 127 -> 166 + 160 us).
-bool gb_shared_ok(const mi_moe_ctx *c, const mi_moe_layer *L, int64_t T) {
-    if (!is_b32f(L->gate.type) || !gb_path(c, L, T)) return false;
+bool b32_shared_ok(const mi_moe_ctx *c, const mi_moe_layer *L, int64_t T) {
+    if (!is_b32f(L->gate.type)) return false;
     if (L->sh_gate.type != L->gate.type || L->sh_down.type != L->down.type || L->sh_act != L->act) return false;
+    if (!gb_path(c, L, T)) return T <= GV_SHARED_T;
     if (!gb_strides_ok(L->sh_gate) || !gb_strides_ok(L->sh_down) || (act_gated(L->act) && !gb_strides_ok(L->sh_up)))
         return false;
     const int64_t K = L->n_expert_used;
@@ -582,11 +588,12 @@ bool gb_shared_ok(const mi_moe_ctx *c, const mi_moe_layer *L, int64_t T) {
 // rows into the combine.  Below the GEMM threshold the grouped GEMV
 // (k_b32.hip), GLU rows in fp32; above it the grouped MFMA GEMM (k_gb.hip),
 // whose gate/up launch writes the down product's operand rows itself.
-// Arguments as run_experts; sh_here: the shared expert too (gb_shared_ok),
+// Arguments as run_experts; sh_here: the shared expert too (b32_shared_ok),
 // its rows' weights in sh_w (NULL: 1), added to the routed sum.
 int run_experts_b32(mi_moe_ctx *c, const mi_moe_layer *L, const float *x, int64_t T, const int32_t *ids_gu,
                     const int32_t *ids_dn, const float *w, const float *res, float *out, hipStream_t st,
-                    bool check_ids, const float *add, bool sh_here = false, const float *sh_w = nullptr) {
+                    bool check_ids, const float *add, bool disp_out = true, bool sh_here = false,
+                    const float *sh_w = nullptr) {
     const int D = L->n_embd, E = L->n_expert, K = L->n_expert_used, I = L->n_ff;
     const int64_t rows = T * K;
     const int max_active = (int)std::min<int64_t>(E, rows);
@@ -608,22 +615,26 @@ int run_experts_b32(mi_moe_ctx *c, const mi_moe_layer *L, const float *x, int64_
     }
     const int bm = gemm ? gb_bm(c, rows, E, D) : G4_BM;
     const int max_tiles = (int)((rows + bm - 1) / bm + max_active);
-    TRY(launch_dispatch(ids_gu, T, K, E, bm, 1, c->disp[0].view(), st));
-    if (!same_ids) TRY(launch_dispatch(ids_dn, T, K, E, bm, 1, c->disp[1].view(), st));
+    // The GEMV's work-groups find their rows from the router's ids themselves
+    // (k_b32.hip), unless the caller wants the dispatch's outputs.
+    const bool self_disp = !gemm && same_ids && !check_ids && !disp_out && rows <= GV_SD_IDS;
+    if (!self_disp) {
+        TRY(launch_dispatch(ids_gu, T, K, E, bm, 1, c->disp[0].view(), st));
+        if (!same_ids) TRY(launch_dispatch(ids_dn, T, K, E, bm, 1, c->disp[1].view(), st));
+    }
     const DispBuf &dg = c->disp[0];
     const DispBuf &dd = same_ids ? c->disp[0] : c->disp[1];
     stage_end(c, "dispatch", st);
     // an activation set in the operand form of a consumer type on this path
-    auto prep_for = [&](int wtype, ActBuf &ab, int64_t width, int pre_act) {
+    auto prep_for = [&](int wtype, ActBuf &ab, int64_t width) {
         B32Prep o;
-        o.pre_act = pre_act;
         o.ldo = gemm ? round_up(width, 64) : width;
         if (wtype == MI_TYPE_F16) { o.mode = B32_PREP_F16; o.xh = ab.h; }
         else if (gemm) { o.mode = B32_PREP_DQ; o.xh = ab.h; }
-        else { o.mode = B32_PREP_CODES; o.q8 = ab.q8; o.dh = (uint16_t *)ab.bs; }
+        else { o.mode = B32_PREP_CODES; o.q8 = ab.q8; o.ds = (uint32_t *)ab.bs; }
         return o;
     };
-    TRY(launch_prep_b32(x, D, T, D, prep_for(L->gate.type, c->ax, D, 0), st));
+    TRY(launch_prep_b32(x, D, T, D, prep_for(L->gate.type, c->ax, D), st));
     stage_end(c, "q8_x", st);
     if (gemm) {
         GBArgs a = {};
@@ -664,24 +675,41 @@ int run_experts_b32(mi_moe_ctx *c, const mi_moe_layer *L, const float *x, int64_
         auto args_for = [&](const ExpertMat &a, const DispBuf &d, const ActBuf &ab, int ne11) {
             B32Args g = {};
             g.a = a; g.ne11 = ne11; g.K = K; g.act = L->act; g.I = I;
-            g.q8 = ab.q8; g.dh = (const uint16_t *)ab.bs; g.xh = ab.h;
+            g.q8 = ab.q8; g.ds = (const uint32_t *)ab.bs; g.xh = ab.h;
             g.counts = d.counts; g.offsets = d.offsets; g.perm = d.perm; g.active_e = d.active_e;
             g.n_active = d.n_active; g.max_active = max_active;
+            if (self_disp) { g.ids = ids_gu; g.rows = rows; }
             return g;
         };
         B32Args a = args_for(as_mat(L->gate), dg, c->ax, 1);
         if (gated && !L->fused_gate_up) a.b = as_mat(L->up);
-        a.glu = gated ? 1 : 0;
-        a.fused = L->fused_gate_up;
-        a.y = c->f1; a.ldy = I; a.ncols = I;
+        a.glu = gated ? 1 : 0; a.relu_sqr = gated ? 0 : 1; a.fused = L->fused_gate_up;
+        a.ncols = I; a.next_f16 = L->down.type == MI_TYPE_F16;
+        a.oq8 = c->aact.q8; a.ods = (uint32_t *)c->aact.bs; a.oxh = c->aact.h;
+        if (sh_here) {
+            const int64_t S = L->sh_n_ff;
+            a.sh_rows = T;
+            a.sh.a = as_mat(L->sh_gate);
+            if (gated) a.sh.b = as_mat(L->sh_up);
+            a.sh.I = a.sh.ncols = S;
+            a.sh.q8 = a.q8; a.sh.ds = a.ds; a.sh.xh = a.xh;
+            // (f1 is free on this path, and holds 2 cap_I floats per slot)
+            a.sh.oxh = (_Float16 *)c->f1;
+            a.sh.oq8 = (int8_t *)c->f1;
+            a.sh.ods = (uint32_t *)((int8_t *)c->f1 + T * S);
+        }
         TRY(launch_gemv_b32(a, st));
         stage_end(c, "gate_up", st);
-        // one product (relu^2 experts): its rows are squared on the way to the down operand
-        TRY(launch_prep_b32(c->f1, I, rows, I, prep_for(L->down.type, c->aact, I, gated ? 0 : MI_ACT_RELU_SQR), st));
-        stage_end(c, "q8_act", st);
         B32Args d = args_for(as_mat(L->down), dd, c->aact, K);
-        d.glu = 0;
         d.y = c->z; d.ldy = D; d.ncols = D;
+        if (sh_here) {
+            d.sh_rows = T;
+            d.sh.a = as_mat(L->sh_down);
+            d.sh.q8 = a.sh.oq8; d.sh.ds = a.sh.ods; d.sh.xh = a.sh.oxh;
+            d.sh.y = c->sh_out; d.sh.ldy = d.sh.ncols = D;
+            d.sh_w = sh_w;
+            add = c->sh_out;
+        }
         TRY(launch_gemv_b32(d, st));
     }
     stage_end(c, "down", st);
@@ -702,7 +730,7 @@ int run_experts(mi_moe_ctx *c, const mi_moe_layer *L, const float *x, int64_t T,
                 bool x_done = false, bool check_ids = false, const float *add = nullptr,
                 bool disp_out = true, bool sh_here = false, const float *sh_w = nullptr) {
     if (is_b32f(L->gate.type))
-        return run_experts_b32(c, L, x, T, ids_gu, ids_dn, w, res, out, st, check_ids, add, sh_here, sh_w);
+        return run_experts_b32(c, L, x, T, ids_gu, ids_dn, w, res, out, st, check_ids, add, disp_out, sh_here, sh_w);
     const int D = L->n_embd, E = L->n_expert, K = L->n_expert_used, I = L->n_ff;
     const int64_t rows = T * K;
     const int max_active = (int)std::min<int64_t>(E, rows);
@@ -1267,7 +1295,7 @@ int forward_impl(mi_moe_ctx *c, const mi_moe_layer *L, const float *x, int64_t T
     // the shared expert first (its own Q8_K of x; the routed block's follows),
     // unless it rides in the routed launches
     const float *add = nullptr;
-    const bool sh_here = L->sh_n_ff > 0 && gb_shared_ok(c, L, T);
+    const bool sh_here = L->sh_n_ff > 0 && b32_shared_ok(c, L, T);
     if (sh_here) {
         if (L->sh_gate_inp) TRY(shared_weights(c, L, x, T, st));
     } else if (L->sh_n_ff > 0) {
@@ -1547,7 +1575,7 @@ int mi_mul_mat_id(mi_moe_ctx *c, const mi_tensor *as, const mi_tensor *b, const 
         o.ldo = gb ? ldx : Kin;
         if (as->type == MI_TYPE_F16) { o.mode = B32_PREP_F16; o.xh = c->ax.h; }
         else if (gb) { o.mode = B32_PREP_DQ; o.xh = c->ax.h; }
-        else { o.mode = B32_PREP_CODES; o.q8 = c->ax.q8; o.dh = (uint16_t *)c->ax.bs; }
+        else { o.mode = B32_PREP_CODES; o.q8 = c->ax.q8; o.ds = (uint32_t *)c->ax.bs; }
         TRY(launch_prep_b32(bp, Kin, T * ne11, Kin, o, st));
         if (gb) {
             GBArgs a = {};
@@ -1559,7 +1587,7 @@ int mi_mul_mat_id(mi_moe_ctx *c, const mi_tensor *as, const mi_tensor *b, const 
         }
         B32Args a = {};
         a.a = M; a.glu = 0; a.ne11 = (int)ne11; a.K = (int)n_used;
-        a.q8 = c->ax.q8; a.dh = (const uint16_t *)c->ax.bs; a.xh = c->ax.h;
+        a.q8 = c->ax.q8; a.ds = (const uint32_t *)c->ax.bs; a.xh = c->ax.h;
         a.counts = dsp.counts; a.offsets = dsp.offsets; a.perm = dsp.perm; a.active_e = dsp.active_e;
         a.n_active = dsp.n_active; a.max_active = max_active;
         a.y = (float *)dst->data; a.ldy = N; a.ncols = N;

@@ -30,6 +30,22 @@ __device__ __forceinline__ void b32_q8_codes(const float (&v)[8], int (&q)[8], u
     for (int j = 0; j < 8; ++j) q[j] = (int)roundf(v[j] * id);
 }
 
+// the lane's 8 codes to q8 and (lead: the first lane of the four) the block's
+// word {fp16 d, sum of its 32 codes << 16} to ds
+__device__ __forceinline__ void b32_store_codes(const float (&v)[8], int8_t *q8, uint32_t *ds, bool lead) {
+    int q[8];
+    uint32_t dh;
+    b32_q8_codes(v, q, dh);
+    uint32_t c[2] = {0u, 0u};
+#pragma unroll
+    for (int j = 0; j < 8; ++j) c[j >> 2] |= (uint32_t)(q[j] & 0xff) << (8 * (j & 3));
+    int sum = __builtin_amdgcn_sdot4(0x01010101, (int)c[0], __builtin_amdgcn_sdot4(0x01010101, (int)c[1], 0, false), false);
+    sum += __builtin_amdgcn_update_dpp(0, sum, 0xB1, 0xf, 0xf, true);
+    sum += __builtin_amdgcn_update_dpp(0, sum, 0x4E, 0xf, 0xf, true);
+    *(uint2 *)q8 = make_uint2(c[0], c[1]);
+    if (lead) *ds = dh | (uint32_t)sum << 16;
+}
+
 // the same as fp16(d q)
 __device__ __forceinline__ uint4 b32_q8x8(const float (&v)[8]) {
     int q[8];

@@ -11,11 +11,11 @@
 // times the two fp16 scales, F16 rows exact fp16 x fp16 products.
 //
 //  * quantizers of weight rows (mi_quantize; ggml quantize_row_*_ref),
-//  * the activation pass: Q8_0 codes + fp16 scales (GEMV), fp16(d q) or fp16(x)
+//  * the activation pass: Q8_0 codes + scale words (GEMV), fp16(d q) or fp16(x)
 //    rows (GEMM, and F16's GEMV),
 //  * the grouped GEMV (decode): 8 lanes per weight row, each lane one 32-value
 //    block per 256 values, integer dots on v_dot4_i32_i8 / fp16 pairs on
-//    v_dot2_f32_f16.
+//    v_dot2_f32_f16, the next product's activation pass in its epilogue.
 // The grouped GEMM (prefill) is k_gb.hip.
 //
 // Block layouts (ggml block_q4_0 / q5_0 / q8_0, no padding, so blocks start
@@ -31,58 +31,9 @@
 namespace mimoe {
 
 template <int WT> struct B32Fmt;
-template <> struct B32Fmt<2> { static constexpr int BYTES = 18, WORDS = 5, OFF = 8; };    // Q4_0
-template <> struct B32Fmt<6> { static constexpr int BYTES = 22, WORDS = 6, OFF = 16; };   // Q5_0
-template <> struct B32Fmt<8> { static constexpr int BYTES = 34, WORDS = 9, OFF = 0; };    // Q8_0
-
-// ------------------------------------------------------------------ block loads
-// The WORDS aligned dwords that intersect the block at p (an even address; a
-// block spans WORDS dwords at either alignment).  Every dword read holds at
-// least one byte of the block, so no read leaves the table's pages.
-template <int WT>
-__device__ inline void b32_words(const uint8_t *p, uint32_t (&w)[B32Fmt<WT>::WORDS], uint32_t &mis) {
-    const uintptr_t a = (uintptr_t)p;
-    mis = (uint32_t)(a & 2u);
-    const uint32_t *q = (const uint32_t *)(a - mis);
-#pragma unroll
-    for (int i = 0; i < B32Fmt<WT>::WORDS; ++i) w[i] = q[i];
-}
-// the 4 block bytes from byte offset OFF (even): bytes [mis + OFF, ...) of
-// the words (compile-time word indices keep the words in registers)
-template <int OFF, int N>
-__device__ inline uint32_t b32_dword(const uint32_t (&w)[N], uint32_t mis) {
-    constexpr int k = OFF >> 2;   // OFF % 4 is 0 or 2
-    if constexpr ((OFF & 2) == 0) return mis ? __builtin_amdgcn_alignbyte(w[k + 1], w[k], 2) : w[k];
-    else return mis ? w[k + 1] : __builtin_amdgcn_alignbyte(w[k + 1], w[k], 2);
-}
-__device__ inline float b32_d(uint32_t w0, uint32_t mis) {
-    return fp16_bits_to_f32(mis ? (w0 >> 16) : (w0 & 0xffffu));
-}
-
-// signed codes of values 4i .. 4i + 3 of the block as bytes, i < 8 (Q8_0:
-// the codes; Q4_0 / Q5_0: the unsigned codes q, the offset is applied by the
-// caller through the block's activation sum)
-template <int WT, int I>
-__device__ inline uint32_t b32_codes4(const uint32_t (&w)[B32Fmt<WT>::WORDS], uint32_t mis) {
-    if constexpr (WT == 8) {
-        return b32_dword<2 + 4 * I>(w, mis);
-    } else {
-        constexpr int QS = WT == 2 ? 2 : 6;
-        const uint32_t qs = b32_dword<QS + 4 * (I & 3)>(w, mis);
-        uint32_t v = I < 4 ? (qs & 0x0F0F0F0Fu) : ((qs >> 4) & 0x0F0F0F0Fu);
-        if constexpr (WT == 6) {
-            const uint32_t qh = b32_dword<2>(w, mis);
-            const uint32_t b = (qh >> (4 * I)) & 0xFu;   // 5th bits of values 4I .. 4I + 3
-            v |= ((b & 1u) << 4) | ((b & 2u) << 11) | ((b & 4u) << 18) | ((b & 8u) << 25);
-        }
-        return v;
-    }
-}
-template <int WT, int I = 0>
-__device__ inline void b32_codes_all(const uint32_t (&w)[B32Fmt<WT>::WORDS], uint32_t mis, uint32_t (&c)[8]) {
-    c[I] = b32_codes4<WT, I>(w, mis);
-    if constexpr (I < 7) b32_codes_all<WT, I + 1>(w, mis, c);
-}
+template <> struct B32Fmt<2> { static constexpr int BYTES = 18, WORDS = 5; };   // Q4_0
+template <> struct B32Fmt<6> { static constexpr int BYTES = 22, WORDS = 6; };   // Q5_0
+template <> struct B32Fmt<8> { static constexpr int BYTES = 34, WORDS = 9; };   // Q8_0
 
 // ------------------------------------------------------------------ quantizers
 // One thread per 32-value block, the oracle's statement order (the scale and
@@ -157,7 +108,7 @@ int launch_quantize_b32(int type, const float *src, void *dst, int64_t nblocks, 
 
 // ------------------------------------------------------------------ activations
 // Rows of K values (K % 32 == 0, row r at src + r * ld) into the operand form
-// of a consumer weight type (B32Prep): Q8_0 codes [r][K] and fp16 scales
+// of a consumer weight type (B32Prep): Q8_0 codes [r][K] and scale words
 // [r][K/32] (GEMV of Q4_0 / Q5_0 / Q8_0), fp16(d q) rows [r][ldo] (their GEMM),
 // or fp16(x) rows [r][ldo] (F16, both paths); the Q8_0 scale and codes are the
 // oracle's bit for bit.  Memory-bound; 8 values per thread, four threads per
@@ -184,22 +135,8 @@ __global__ void __launch_bounds__(256) k_prep_b32(const float *src, int64_t ld, 
 #pragma unroll
         for (int j = 0; j < 8; ++j) v[j] = 0.f;
     }
-    if (o.pre_act == 4) {   // ggml_sqr(ggml_relu(u)) before the quantization
-#pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = relu_sqr(v[j]);
-    }
     if (o.mode == B32_PREP_CODES) {
-        int q[8];
-        uint32_t dh;
-        b32_q8_codes(v, q, dh);
-        uint32_t lo = 0, hi = 0;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            lo |= (uint32_t)(q[j] & 0xff) << (8 * j);
-            hi |= (uint32_t)(q[4 + j] & 0xff) << (8 * j);
-        }
-        *(uint2 *)(o.q8 + r * K + 8 * c) = make_uint2(lo, hi);
-        if ((c & 3) == 0) o.dh[r * (K / 32) + c / 4] = (uint16_t)dh;
+        b32_store_codes(v, o.q8 + r * K + 8 * c, o.ds + r * (K / 32) + c / 4, (c & 3) == 0);
     } else {
         *(uint4 *)(o.xh + r * o.ldo + 8 * c) = o.mode == B32_PREP_F16 ? b32_f16x8(v) : b32_q8x8(v);
     }
@@ -218,107 +155,316 @@ int launch_prep_b32(const float *src, int64_t ld, int64_t nrows, int64_t K, cons
 }
 
 // ------------------------------------------------------------------ GEMV
-// dot of one 32-value block (this lane's) with the activation row's block
+// One block (32 values) of a weight row in registers (blocks start at any even byte)
+template <int WT> struct GvBlk { uint32_t w[B32Fmt<WT>::WORDS]; };
+template <> struct GvBlk<1> { uint4 v[4]; };
+
+// the WORDS dwords from the dword at or below the block's first byte: each
+// holds at least one byte of the block, so no read leaves the table's pages
 template <int WT>
-__device__ inline float b32_block_dot(const uint8_t *wblk, const int8_t *xq, float dx) {
-    uint32_t w[B32Fmt<WT>::WORDS], mis;
-    b32_words<WT>(wblk, w, mis);
-    const uint4 xa = *(const uint4 *)xq, xb = *(const uint4 *)(xq + 16);
-    const uint32_t xv[8] = {xa.x, xa.y, xa.z, xa.w, xb.x, xb.y, xb.z, xb.w};
-    uint32_t cw[8];
-    b32_codes_all<WT>(w, mis, cw);
-    int isum = 0, xsum = 0;
+__device__ __forceinline__ void gv_load(const uint8_t *p, GvBlk<WT> &o) {
+    if constexpr (WT == 1) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        isum = __builtin_amdgcn_sdot4((int)cw[i], (int)xv[i], isum, false);
-        if constexpr (WT != 8) xsum = __builtin_amdgcn_sdot4(0x01010101, (int)xv[i], xsum, false);
+        for (int c = 0; c < 4; ++c) o.v[c] = *(const uint4 *)(p + 16 * c);
+    } else {
+        const uint8_t *q = p - ((uintptr_t)p & 2u);
+        __builtin_memcpy(o.w, __builtin_assume_aligned(q, 4), 4 * B32Fmt<WT>::WORDS);
     }
-    const float dw = b32_d(w[0], mis);
-    // the expression orders of ggml_vec_dot_q{4,5,8}_0_q8_0
-    if constexpr (WT == 8) return (float)isum * (dw * dx);
-    else if constexpr (WT == 6) return (dw * dx) * (float)(isum - 16 * xsum);
-    else return (float)(isum - 8 * xsum) * dw * dx;
 }
 
-__device__ inline float f16_block_dot(const uint8_t *wblk, const _Float16 *xh) {
-    float acc = 0.f;
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        const uint4 wv = *(const uint4 *)(wblk + 16 * c);
-        const uint4 xv = *(const uint4 *)(xh + 8 * c);
-        const uint32_t wa[4] = {wv.x, wv.y, wv.z, wv.w}, xa[4] = {xv.x, xv.y, xv.z, xv.w};
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            acc = __builtin_amdgcn_fdot2(__builtin_bit_cast(half2_t, wa[i]), __builtin_bit_cast(half2_t, xa[i]),
-                                         acc, false);
-    }
-    return acc;
-}
-
-// Grid (column blocks, active experts), 4 waves of 8 row groups x 8 lanes; a
-// row group owns one weight row (GLU: groups 0-3 the gate rows, 4-7 the
-// matching up rows), lane sl takes blocks sl, sl + 8, ... of it for every
-// token of the expert (the row's bytes come from HBM once, from the caches
-// for the later tokens).
+// the block's codes, 4 to a dword in value order (Q4_0 / Q5_0: unsigned; F16: the values), and its scale;
+// mis: 2 where the block starts in the middle of a dword, else 0
 template <int WT>
-__global__ void __launch_bounds__(256) k_gemv_b32(B32Args g) {
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int rs = lane >> 3, sl = lane & 7;
-    const int j = blockIdx.y;
-    if (j >= *g.n_active) return;
-    const int e = g.active_e[j];
-    const int cnt = g.counts[e], off = g.offsets[e];
-    const bool glu = g.glu != 0;
-    const int64_t col0 = ((int64_t)blockIdx.x * 4 + wave) * (glu ? 4 : 8);
-    int64_t col = col0 + (glu ? (rs & 3) : rs);
-    const bool col_ok = col < g.ncols;
-    if (!col_ok) col = 0;
-    const ExpertMat *M = &g.a;
-    int64_t wrow = col;
-    if (glu && rs >= 4) {
-        if (g.fused) wrow = g.I + col;
-        else M = &g.b;
-    }
-    const uint8_t *rowp = M->data + (int64_t)e * M->mat_bytes + wrow * M->row_bytes;
-    const int64_t Kin = M->K, nbr = Kin / 32;
-    for (int m = 0; m < cnt; ++m) {
-        const int p = g.perm[off + m];
-        const int64_t arow = g.ne11 == 1 ? p / g.K : p;
-        float acc = 0.f;
-        for (int64_t b = sl; b < nbr; b += 8) {
-            if constexpr (WT == 1) {
-                acc += f16_block_dot(rowp + 64 * b, g.xh + arow * Kin + 32 * b);
-            } else {
-                const float dx = fp16_bits_to_f32(g.dh[arow * nbr + b]);
-                acc += b32_block_dot<WT>(rowp + (int64_t)B32Fmt<WT>::BYTES * b, g.q8 + arow * Kin + 32 * b, dx);
+__device__ __forceinline__ float gv_codes(const GvBlk<WT> &o, uint32_t mis, uint32_t (&c)[8]) {
+    constexpr int NW = B32Fmt<WT>::WORDS;
+    // bytes 2 + 4 i .. of the block: from word i (mis 0) or i + 1
+    auto after = [&](int i) __attribute__((always_inline)) {
+        const uint32_t hi = i + 1 < NW ? o.w[i + 1] : 0u;
+        return mis ? hi : __builtin_amdgcn_alignbyte(hi, o.w[i], 2);
+    };
+    const float d = fp16_bits_to_f32(mis ? o.w[0] >> 16 : o.w[0] & 0xffffu);
+    if constexpr (WT == 8) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) c[i] = after(i);
+    } else {
+        constexpr int O = WT == 6 ? 1 : 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t q = after(i + O);
+            c[i] = q & 0x0F0F0F0Fu;
+            c[4 + i] = (q >> 4) & 0x0F0F0F0Fu;
+        }
+        if constexpr (WT == 6) {
+            const uint32_t qh = after(0);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                // fifth bits of 4 values, bit j to bit 8 j (four copies 7 bits apart, no carry), then to bit 4
+                const uint32_t b = (qh >> (4 * i)) & 0xFu;
+                c[i] |= (__umul24(b, 0x204081u) & 0x01010101u) << 4;
             }
         }
-        acc += __shfl_xor(acc, 1, 64);
-        acc += __shfl_xor(acc, 2, 64);
-        acc += __shfl_xor(acc, 4, 64);
-        if (glu) {
-            const float other = __shfl(acc, lane + 32 < 64 ? lane + 32 : lane, 64);
-            if (rs < 4 && sl == 0 && col_ok) g.y[(int64_t)p * g.ldy + col] = act_pair(g.act, acc, other);
+    }
+    return d;
+}
+
+// LDS of a pass: the activation blocks of up to GV_NT tokens, GV_KS values of
+// each (quant: codes, then {fp16 scale, sum of the codes} words; F16: values)
+constexpr int GV_NT = 4, GV_KS = 4096, GV_WAVES = 8;
+template <int WT> constexpr int gv_row() { return WT == 1 ? 2 * GV_KS : GV_KS + GV_KS / 8; }
+
+// acc[n] += the lane's blocks sl, sl + 8, ... of its weight row times tokens
+// n0 .. n0 + NT - 1 (rows s_p[n0 + n], clamped to the last), block by block
+template <int WT, int NT>
+__device__ __forceinline__ void gv_pass(const B32Side &s, int kdiv, const uint8_t *rowp, const int *s_p, int n0, int cnt,
+                                        uint8_t *xs, float (&acc)[GV_NT], int sl, int tid) {
+    constexpr int U = WT != 1 && NT == 1 ? 4 : 2;   // blocks in flight per lane
+    constexpr int BB = WT == 1 ? 64 : B32Fmt<WT == 1 ? 8 : WT>::BYTES, ROW = gv_row<WT>();
+    const int K = (int)s.a.K, nbr = K / 32;
+#pragma unroll
+    for (int n = 0; n < GV_NT; ++n) acc[n] = 0.f;
+    for (int k0 = 0; k0 < nbr; k0 += GV_KS / 32) {
+        const int nb = nbr - k0 < GV_KS / 32 ? nbr - k0 : GV_KS / 32;
+        GvBlk<WT> w[U];
+        auto load = [&](int b) __attribute__((always_inline)) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int bb = b + 8 * u < nb ? b + 8 * u : 0;   // (block 0 again: not used)
+                gv_load<WT>(rowp + (int64_t)BB * (k0 + bb), w[u]);
+            }
+        };
+        load(sl);
+        if (k0 || n0) __syncthreads();   // (the activations before are read)
+#pragma unroll
+        for (int n = 0; n < NT; ++n) {
+            const int p = s_p[n0 + n < cnt ? n0 + n : cnt - 1];
+            const int64_t r = kdiv > 1 ? p / kdiv : p;
+            uint8_t *o = xs + n * ROW;
+            if constexpr (WT == 1) {
+                const uint8_t *src = (const uint8_t *)(s.xh + r * K + 32 * k0);
+                for (int i = tid; i < 4 * nb; i += 64 * GV_WAVES) *(uint4 *)(o + 16 * i) = *(const uint4 *)(src + 16 * i);
+            } else {
+                const uint8_t *src = (const uint8_t *)(s.q8 + r * K + 32 * k0);
+                for (int i = tid; i < 2 * nb; i += 64 * GV_WAVES) *(uint4 *)(o + 16 * i) = *(const uint4 *)(src + 16 * i);
+                const uint32_t *sd = s.ds + r * nbr + k0;
+                for (int i = tid; i < nb; i += 64 * GV_WAVES) *(uint32_t *)(o + GV_KS + 4 * i) = sd[i];
+            }
+        }
+        __syncthreads();
+        for (int b0 = sl; b0 < nb; b0 += 8 * U) {
+            if (b0 != sl) load(b0);
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int b = b0 + 8 * u;
+                if (b >= nb) break;
+                if constexpr (WT == 1) {
+#pragma unroll
+                    for (int n = 0; n < NT; ++n) {
+                        float d = 0.f;
+#pragma unroll
+                        for (int c = 0; c < 4; ++c) {
+                            const uint4 xv = *(const uint4 *)(xs + (n * ROW + 64 * b + 16 * c));
+                            const uint32_t wa[4] = {w[u].v[c].x, w[u].v[c].y, w[u].v[c].z, w[u].v[c].w};
+                            const uint32_t xa[4] = {xv.x, xv.y, xv.z, xv.w};
+#pragma unroll
+                            for (int i = 0; i < 4; ++i)
+                                d = __builtin_amdgcn_fdot2(__builtin_bit_cast(half2_t, wa[i]), __builtin_bit_cast(half2_t, xa[i]),
+                                                           d, false);
+                        }
+                        acc[n] += d;
+                    }
+                } else {
+                    uint32_t c[8];
+                    const float dw = gv_codes<WT>(w[u], (uint32_t)(uintptr_t)(rowp + (int64_t)BB * (k0 + b)) & 2u, c);
+#pragma unroll
+                    for (int n = 0; n < NT; ++n) {
+                        const uint4 xa = *(const uint4 *)(xs + (n * ROW + 32 * b)), xb = *(const uint4 *)(xs + (n * ROW + 32 * b + 16));
+                        const uint32_t ds = *(const uint32_t *)(xs + (n * ROW + GV_KS + 4 * b));
+                        const uint32_t xv[8] = {xa.x, xa.y, xa.z, xa.w, xb.x, xb.y, xb.z, xb.w};
+                        int isum = 0;
+#pragma unroll
+                        for (int i = 0; i < 8; ++i) isum = __builtin_amdgcn_sdot4((int)c[i], (int)xv[i], isum, false);
+                        const float dx = fp16_bits_to_f32(ds & 0xffffu);
+                        const int xsum = (int)ds >> 16;
+                        // the expression orders of ggml_vec_dot_q{4,5,8}_0_q8_0
+                        if constexpr (WT == 8) acc[n] += (float)isum * (dw * dx);
+                        else if constexpr (WT == 6) acc[n] += (dw * dx) * (float)(isum - 16 * xsum);
+                        else acc[n] += (float)(isum - 8 * xsum) * dw * dx;
+                    }
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+        acc[n] += __shfl_xor(acc[n], 1, 64);
+        acc[n] += __shfl_xor(acc[n], 2, 64);
+        acc[n] += __shfl_xor(acc[n], 4, 64);
+    }
+}
+
+// A work-group (8 waves) owns 64 weight rows of one active expert (GLU: 32
+// gate rows and the matching up rows), a wave 8 row groups x 8 lanes (GLU:
+// groups 0-3 gate, 4-7 up); lane sl takes blocks sl, sl + 8, ... of its row.
+// The expert's tokens run four to a pass through LDS, a weight block decoded
+// once for the four.
+//
+// The gate/up form writes the down product's operand itself (a GLU
+// work-group's 32 columns are one Q8_0 block of each row), the bits of
+// launch_prep_b32 on the fp32 values.  With g.ids the expert list comes from
+// the ids: work-group row j belongs to slot j, and leaves unless the slot is
+// its expert's first.  SH: the shared expert's work-groups come first.
+//
+// What bounds it: the load path (a block is 2 - 3 loads of at most 16 bytes
+// at dword-aligned addresses; the same bytes at their own, 2-byte aligned
+// addresses: moondream3 Q8_0 T = 5 gate/up 36.7 against 31.2 us, down 24.5
+// against 19.8) and the work-groups in flight (four blocks ahead with one
+// token in the pass, two with more: at 125 registers 16 waves per CU; eight
+// ahead spills, 24 - 32 waves per CU with two tokens a pass are slower for
+// many rows).  Against the form before (each lane reading its blocks dword by
+// dword and the activations from the caches for every token anew, the GLU
+// rows quantized by a launch of their own, a dispatch launch, the shared
+// expert as a layer of its own), layer us: moondream3 Q8_0 T = 1 / 5 47.6 /
+// 78.5 -> 37 / 71, Q4_0 T = 5 72 -> 62; qwen3omni Q5_0 T = 12 127 -> 101,
+// Q8_0 T = 16 150 -> 131; nemotronomni Q5_0 T = 1 / 4 / 16 109 / 177 / 302 ->
+// 47 / 80 / 176; diffusiongemma F16 T = 4 / 16 104 / 273 -> 95 / 203.
+enum { GV_STORE = 0, GV_GLU = 1, GV_RELU_SQR = 2 };
+template <int WT, int EPI, bool SH>
+__global__ void __launch_bounds__(64 * GV_WAVES) __attribute__((amdgpu_waves_per_eu(4))) k_gemv_b32(B32Args g) {
+    __shared__ __attribute__((aligned(16))) uint8_t xs[GV_NT * gv_row<WT>()];
+    __shared__ float s_v[GV_NT][64];
+    __shared__ int s_p[GV_SD_IDS];
+    __shared__ int s_cnt[GV_WAVES];
+    constexpr bool GLU = EPI == GV_GLU;
+    constexpr int COLS = GLU ? 32 : 64;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int rs = lane >> 3, sl = lane & 7;
+    const bool shared = SH && (int)blockIdx.x < g.sh_wgs;
+    const B32Side s = shared ? g.sh : (const B32Side &)g;
+    int e = 0, cnt, cb;
+    const int32_t *perm = nullptr;   // the rows (null: in s_p)
+    if (shared) {
+        cb = blockIdx.x;
+        cnt = (int)g.sh_rows;
+    } else {
+        const unsigned lin = blockIdx.x - (SH ? g.sh_wgs : 0), j = lin / (unsigned)g.ncb;
+        cb = (int)(lin - j * (unsigned)g.ncb);
+        if (g.ids) {
+            const int id = tid < g.rows ? g.ids[tid] : -1;
+            e = g.ids[j];
+            const uint64_t m = __ballot(id == e);
+            if (lane == 0) s_cnt[wave] = __popcll(m);
+            __syncthreads();
+            int before = 0, total = 0;
+#pragma unroll
+            for (int i = 0; i < GV_WAVES; ++i) {
+                if (i < wave) before += s_cnt[i];
+                total += s_cnt[i];
+            }
+            if (id == e) s_p[before + __popcll(m & ((1ull << lane) - 1))] = tid;
+            __syncthreads();
+            if (s_p[0] != (int)j) return;
+            cnt = total;
         } else {
-            if (sl == 0 && col_ok) g.y[(int64_t)p * g.ldy + col] = acc;
+            if ((int)j >= *g.n_active) return;
+            e = g.active_e[j];
+            cnt = g.counts[e];
+            perm = g.perm + g.offsets[e];
+        }
+    }
+    const int64_t col = (int64_t)cb * COLS + wave * (COLS / GV_WAVES) + (GLU ? (rs & 3) : rs);
+    const bool col_ok = col < s.ncols;
+    int64_t wrow = col_ok ? col : 0;
+    const uint8_t *rowp = s.a.data + (int64_t)e * s.a.mat_bytes;
+    int64_t rb = s.a.row_bytes;
+    if (GLU && rs >= 4) {
+        if (s.fused) {
+            wrow += s.I;
+        } else {
+            rowp = s.b.data + (int64_t)e * s.b.mat_bytes;
+            rb = s.b.row_bytes;
+        }
+    }
+    rowp += wrow * rb;
+    const int kdiv = g.ne11 == 1 && !shared ? g.K : 1;
+    for (int q0 = 0; q0 < cnt; q0 += GV_SD_IDS) {   // (rows that fit s_p)
+        const int qn = cnt - q0 < GV_SD_IDS ? cnt - q0 : GV_SD_IDS;
+        if (shared || perm) {
+            if (q0) __syncthreads();
+            for (int i = tid; i < qn; i += 64 * GV_WAVES) s_p[i] = shared ? q0 + i : perm[q0 + i];
+            __syncthreads();
+        }
+        for (int n0 = 0; n0 < qn; n0 += GV_NT) {
+            const int nt = qn - n0 < GV_NT ? qn - n0 : GV_NT;
+            float acc[GV_NT];
+            if (nt == 1) gv_pass<WT, 1>(s, kdiv, rowp, s_p, n0, qn, xs, acc, sl, tid);
+            else if (nt == 2) gv_pass<WT, 2>(s, kdiv, rowp, s_p, n0, qn, xs, acc, sl, tid);
+            else gv_pass<WT, GV_NT>(s, kdiv, rowp, s_p, n0, qn, xs, acc, sl, tid);
+            if constexpr (EPI == GV_STORE) {
+#pragma unroll
+                for (int n = 0; n < GV_NT; ++n) {
+                    if (n >= nt || sl != 0 || !col_ok) continue;
+                    const int p = s_p[n0 + n];
+                    s.y[(int64_t)p * s.ldy + col] = shared && g.sh_w ? acc[n] * g.sh_w[p] : acc[n];
+                }
+            } else {
+#pragma unroll
+                for (int n = 0; n < GV_NT; ++n) {
+                    if (n >= nt) continue;
+                    const float other = GLU ? __shfl(acc[n], (lane + 32) & 63, 64) : 0.f;
+                    if (sl == 0 && (!GLU || rs < 4))
+                        s_v[n][wave * (COLS / GV_WAVES) + rs] = GLU ? act_pair(g.act, acc[n], other) : relu_sqr(acc[n]);
+                }
+                __syncthreads();
+                const int n = tid / (COLS / 8), c8 = tid % (COLS / 8);   // 8 values per thread, four threads per block
+                const int64_t c0 = (int64_t)cb * COLS + 8 * c8;
+                if (n < nt && c0 < s.ncols) {
+                    float v[8];
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) v[i] = s_v[n][8 * c8 + i];
+                    const int64_t p = s_p[n0 + n];
+                    if (g.next_f16) *(uint4 *)(s.oxh + p * s.ncols + c0) = b32_f16x8(v);
+                    else b32_store_codes(v, s.oq8 + p * s.ncols + c0, s.ods + p * (s.ncols / 32) + c0 / 32, (c8 & 3) == 0);
+                }
+                // (s_v is written again after the barrier in front of the next pass's products)
+            }
         }
     }
 }
 
 // ------------------------------------------------------------------ launch
+template <int WT, int EPI>
+static int gv_launch(const B32Args &a, hipStream_t st) {
+    B32Args g = a;
+    constexpr int COLS = EPI == GV_GLU ? 32 : 64;
+    g.ncb = (int)((g.ncols + COLS - 1) / COLS);
+    g.sh_wgs = g.sh_rows > 0 ? (int)((g.sh.ncols + COLS - 1) / COLS) : 0;
+    const int64_t wgs = g.sh_wgs + (int64_t)g.ncb * (g.ids ? g.rows : g.max_active);
+    if (wgs > 0x7fffffff) return -6;
+    const dim3 grid((unsigned)wgs), block(64 * GV_WAVES);
+    if (g.sh_wgs) hipLaunchKernelGGL((k_gemv_b32<WT, EPI, true>), grid, block, 0, st, g);
+    else hipLaunchKernelGGL((k_gemv_b32<WT, EPI, false>), grid, block, 0, st, g);
+    return hip_check_launch();
+}
+
 int launch_gemv_b32(const B32Args &g, hipStream_t st) {
     if (g.max_active <= 0) return 0;
-    if (g.a.K % 32) return -6;
-    const int64_t per_block = (g.glu ? 4 : 8) * 4;
-    const dim3 grid((unsigned)((g.ncols + per_block - 1) / per_block), (unsigned)g.max_active);
+    if (g.a.K % 32 || g.a.K > 0x7fffffff) return -6;
+    if (g.ids && g.rows > GV_SD_IDS) return -6;
+    if ((g.glu || g.relu_sqr) && g.ncols % 32) return -6;
+    if (g.sh_rows > 0 && (g.sh.a.type != g.a.type || g.sh.a.K % 32 || ((g.glu || g.relu_sqr) && g.sh.ncols % 32))) return -6;
+#define GV_TYPE(T)                                                \
+    case T:                                                       \
+        if (g.glu) return gv_launch<T, GV_GLU>(g, st);            \
+        if (g.relu_sqr) return gv_launch<T, GV_RELU_SQR>(g, st);  \
+        return gv_launch<T, GV_STORE>(g, st);
     switch (g.a.type) {
-    case 1: hipLaunchKernelGGL(k_gemv_b32<1>, grid, dim3(256), 0, st, g); break;
-    case 2: hipLaunchKernelGGL(k_gemv_b32<2>, grid, dim3(256), 0, st, g); break;
-    case 6: hipLaunchKernelGGL(k_gemv_b32<6>, grid, dim3(256), 0, st, g); break;
-    case 8: hipLaunchKernelGGL(k_gemv_b32<8>, grid, dim3(256), 0, st, g); break;
+        GV_TYPE(1)
+        GV_TYPE(2)
+        GV_TYPE(6)
+        GV_TYPE(8)
     default: return -3;
     }
-    return hip_check_launch();
+#undef GV_TYPE
 }
 
 }  // namespace mimoe

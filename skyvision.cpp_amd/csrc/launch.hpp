@@ -257,25 +257,44 @@ struct B32Prep {
     int mode;                  // CODES: Q8_0 codes + scales (GEMV of Q4_0/Q5_0/Q8_0); DQ: fp16(d q) rows
                                // (their GEMM); F16: fp16(x) rows (F16 tables, both paths)
     int8_t *q8 = nullptr;      // CODES: [rows][K]
-    uint16_t *dh = nullptr;    // CODES: [rows][K/32] fp16 scale bits
+    uint32_t *ds = nullptr;    // CODES: [rows][K/32] {fp16 scale bits, sum of the 32 codes << 16}
     _Float16 *xh = nullptr;    // DQ / F16: [rows][ldo]
     int64_t ldo = 0;           // >= K; values K .. ldo - 1 of a row are written as zeros
-    int pre_act = 0;           // 4 (ACT_RELU_SQR): relu(v)^2 first
 };
 int launch_prep_b32(const float *src, int64_t ld, int64_t nrows, int64_t K, const B32Prep &o, hipStream_t st);
-struct B32Args {
+// Grouped GEMV.  Plain product: fp32 rows y.  glu / relu_sqr: the activation
+// rows leave as the next product's operand (rows of ncols values: fp16 oxh
+// with next_f16, else codes oq8 and words ods; ncols % 32 == 0).  ids: the
+// rows' expert ids, at most GV_SD_IDS of them, in place of the dispatch's
+// lists.  A shared expert (sh_rows > 0) as in GBArgs.
+struct B32Side {
     ExpertMat a, b;            // b: up table (separate gate/up GLU), else unused
-    int glu, fused, act;
+    int fused;
     int64_t I;
     const int8_t *q8;          // Q4_0/Q5_0/Q8_0: Q8_0 codes [rows][K] and
-    const uint16_t *dh;        //   fp16 scales [rows][K/32]
+    const uint32_t *ds;        //   scale words [rows][K/32] (B32Prep)
     const _Float16 *xh;        // F16: fp16 rows [rows][K]
+    float *y;                  // rows p, stride ldy
+    int64_t ldy, ncols;
+    int8_t *oq8;
+    uint32_t *ods;
+    _Float16 *oxh;
+};
+struct B32Args : B32Side {
+    int glu, act;
+    int relu_sqr;              // one product, relu(v)^2 of it
+    int next_f16;
     int ne11, K;
     const int32_t *counts, *offsets, *perm, *active_e, *n_active;
     int max_active;
-    float *y;                  // rows p (glu: act rows [p][I]), stride ldy
-    int64_t ldy, ncols;
+    const int32_t *ids;
+    int64_t rows;
+    B32Side sh;
+    int64_t sh_rows;
+    const float *sh_w;
+    int ncb, sh_wgs;           // (set by launch_gemv_b32)
 };
+constexpr int GV_SD_IDS = 512;
 int launch_gemv_b32(const B32Args &g, hipStream_t st);
 
 // Grouped MFMA GEMM of the same tables (k_gb.hip) on balanced tiles of at

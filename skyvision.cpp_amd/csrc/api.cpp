@@ -583,6 +583,17 @@ bool b32_shared_ok(const mi_moe_ctx *c, const mi_moe_layer *L, int64_t T) {
     return T <= gb_max_tokens(std::max({round_up(L->n_embd, 64), K * round_up(L->n_ff, 64), round_up(L->sh_n_ff, 64)}));
 }
 
+// the operand form of x for the gate/up product
+B32Prep b32_x_prep(const mi_moe_ctx *c, const mi_moe_layer *L, int64_t T) {
+    const bool gemm = gb_path(c, L, T);
+    B32Prep o;
+    o.ldo = gemm ? round_up(L->n_embd, 64) : L->n_embd;
+    if (L->gate.type == MI_TYPE_F16) { o.mode = B32_PREP_F16; o.xh = c->ax.h; }
+    else if (gemm) { o.mode = B32_PREP_DQ; o.xh = c->ax.h; }
+    else { o.mode = B32_PREP_CODES; o.q8 = c->ax.q8; o.ds = (uint32_t *)c->ax.bs; }
+    return o;
+}
+
 // routed FFN body of a layer with Q4_0 / Q5_0 / Q8_0 / F16 tables: the rows
 // converted to each product's ggml vec_dot_type (Q8_0 or fp16), fp32 slot
 // rows into the combine.  Below the GEMM threshold the grouped GEMV
@@ -592,7 +603,7 @@ bool b32_shared_ok(const mi_moe_ctx *c, const mi_moe_layer *L, int64_t T) {
 // its rows' weights in sh_w (NULL: 1), added to the routed sum.
 int run_experts_b32(mi_moe_ctx *c, const mi_moe_layer *L, const float *x, int64_t T, const int32_t *ids_gu,
                     const int32_t *ids_dn, const float *w, const float *res, float *out, hipStream_t st,
-                    bool check_ids, const float *add, bool disp_out = true, bool sh_here = false,
+                    bool x_done, bool check_ids, const float *add, bool disp_out = true, bool sh_here = false,
                     const float *sh_w = nullptr) {
     const int D = L->n_embd, E = L->n_expert, K = L->n_expert_used, I = L->n_ff;
     const int64_t rows = T * K;
@@ -607,7 +618,7 @@ int run_experts_b32(mi_moe_ctx *c, const mi_moe_layer *L, const float *x, int64_
         for (int64_t t0 = 0; t0 < T; t0 += tmax) {
             const int64_t n = std::min(tmax, T - t0);
             TRY(run_experts_b32(c, L, x + t0 * D, n, ids_gu + t0 * K, ids_dn + t0 * K, w + t0 * K,
-                                res ? res + t0 * D : nullptr, out + t0 * D, st, check_ids, add ? add + t0 * D : nullptr));
+                                res ? res + t0 * D : nullptr, out + t0 * D, st, false, check_ids, add ? add + t0 * D : nullptr));
         }
         DispBuf whole = c->disp[0];
         whole.bad_total = nullptr;   // (counted by the passes)
@@ -625,16 +636,7 @@ int run_experts_b32(mi_moe_ctx *c, const mi_moe_layer *L, const float *x, int64_
     const DispBuf &dg = c->disp[0];
     const DispBuf &dd = same_ids ? c->disp[0] : c->disp[1];
     stage_end(c, "dispatch", st);
-    // an activation set in the operand form of a consumer type on this path
-    auto prep_for = [&](int wtype, ActBuf &ab, int64_t width) {
-        B32Prep o;
-        o.ldo = gemm ? round_up(width, 64) : width;
-        if (wtype == MI_TYPE_F16) { o.mode = B32_PREP_F16; o.xh = ab.h; }
-        else if (gemm) { o.mode = B32_PREP_DQ; o.xh = ab.h; }
-        else { o.mode = B32_PREP_CODES; o.q8 = ab.q8; o.ds = (uint32_t *)ab.bs; }
-        return o;
-    };
-    TRY(launch_prep_b32(x, D, T, D, prep_for(L->gate.type, c->ax, D), st));
+    if (!x_done) TRY(launch_prep_b32(x, D, T, D, b32_x_prep(c, L, T), st));
     stage_end(c, "q8_x", st);
     if (gemm) {
         GBArgs a = {};
@@ -730,7 +732,7 @@ int run_experts(mi_moe_ctx *c, const mi_moe_layer *L, const float *x, int64_t T,
                 bool x_done = false, bool check_ids = false, const float *add = nullptr,
                 bool disp_out = true, bool sh_here = false, const float *sh_w = nullptr) {
     if (is_b32f(L->gate.type))
-        return run_experts_b32(c, L, x, T, ids_gu, ids_dn, w, res, out, st, check_ids, add, disp_out, sh_here, sh_w);
+        return run_experts_b32(c, L, x, T, ids_gu, ids_dn, w, res, out, st, x_done, check_ids, add, disp_out, sh_here, sh_w);
     const int D = L->n_embd, E = L->n_expert, K = L->n_expert_used, I = L->n_ff;
     const int64_t rows = T * K;
     const int max_active = (int)std::min<int64_t>(E, rows);
@@ -1311,8 +1313,16 @@ int forward_impl(mi_moe_ctx *c, const mi_moe_layer *L, const float *x, int64_t T
         // router + Q8_K(x) in one launch where the shape fits (the router's
         // own rows: the router alone, the experts quantize x themselves)
         Q8Out qx;
-        const bool xq = !xr && x_q8_spec(c, L, T, qx);
+        bool xq = !xr && x_q8_spec(c, L, T, qx);
         const float *xrow = xr ? xr : x;
+        if (is_b32f(L->gate.type) && front_takes_b32(L->router_w, xrow, D, D, x, D) &&
+            (!gb_path(c, L, T) || T <= gb_max_tokens(std::max(round_up(D, 64), K * round_up(L->n_ff, 64))))) {
+            qx = Q8Out{};
+            qx.b32 = b32_x_prep(c, L, T);
+            qx.b_src = x;
+            qx.b_ld = D;
+            xq = true;
+        }
         Gating gt;
         gt.kind = L->gating;
         gt.sel_bias = L->sel_bias;

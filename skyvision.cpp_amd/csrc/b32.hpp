@@ -5,6 +5,7 @@
 #pragma once
 
 #include "common.hpp"
+#include "launch.hpp"
 #include "wave_ops.hpp"
 
 namespace mimoe {
@@ -61,6 +62,27 @@ __device__ __forceinline__ uint4 b32_q8x8(const float (&v)[8]) {
         h[j] = __builtin_bit_cast(uint32_t, p);
     }
     return make_uint4(h[0], h[1], h[2], h[3]);
+}
+
+// values 8 c .. 8 c + 7 of row r (at x, K values) as o asks
+template <bool VEC>
+__device__ __forceinline__ void b32_prep8(const float *row, int64_t r, int64_t c, int64_t K, const B32Prep &o) {
+    float v[8];
+    if (8 * c < K) {
+        const float *x = row + 8 * c;
+        if constexpr (VEC) {
+            const float4 a = *(const float4 *)x, b = *(const float4 *)(x + 4);
+            v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+        } else {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[j] = x[j];
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = 0.f;
+    }
+    if (o.mode == B32_PREP_CODES) b32_store_codes(v, o.q8 + r * K + 8 * c, o.ds + r * (K / 32) + c / 4, (c & 3) == 0);
+    else *(uint4 *)(o.xh + r * o.ldo + 8 * c) = o.mode == B32_PREP_F16 ? b32_f16x8(v) : b32_q8x8(v);
 }
 
 }  // namespace mimoe

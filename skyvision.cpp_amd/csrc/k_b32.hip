@@ -114,32 +114,16 @@ int launch_quantize_b32(int type, const float *src, void *dst, int64_t nblocks, 
 // oracle's bit for bit.  Memory-bound; 8 values per thread, four threads per
 // block (16-byte loads and stores; 600 rows of 2048: 5.0 us,
 // one value per lane 8.5).
+// Where the router's launch reads the same rows it writes them instead
+// (k_route.hip).
 // VEC: 16-byte aligned rows.
 template <bool VEC>
 __global__ void __launch_bounds__(256) k_prep_b32(const float *src, int64_t ld, int64_t nrows, int64_t K, B32Prep o) {
     const int64_t w = o.mode == B32_PREP_CODES ? K : o.ldo, nch = w / 8;   // 8-value chunks per row (a multiple of 4)
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= nrows * nch) return;   // the four threads of a block leave together
-    const int64_t r = i / nch, c = i - r * nch;
-    float v[8];
-    if (8 * c < K) {
-        const float *x = src + r * ld + 8 * c;
-        if constexpr (VEC) {
-            const float4 a = *(const float4 *)x, b = *(const float4 *)(x + 4);
-            v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-        } else {
-#pragma unroll
-            for (int j = 0; j < 8; ++j) v[j] = x[j];
-        }
-    } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = 0.f;
-    }
-    if (o.mode == B32_PREP_CODES) {
-        b32_store_codes(v, o.q8 + r * K + 8 * c, o.ds + r * (K / 32) + c / 4, (c & 3) == 0);
-    } else {
-        *(uint4 *)(o.xh + r * o.ldo + 8 * c) = o.mode == B32_PREP_F16 ? b32_f16x8(v) : b32_q8x8(v);
-    }
+    const int64_t r = i / nch;
+    b32_prep8<VEC>(src + r * ld, r, i - r * nch, K, o);
 }
 
 int launch_prep_b32(const float *src, int64_t ld, int64_t nrows, int64_t K, const B32Prep &o, hipStream_t st) {

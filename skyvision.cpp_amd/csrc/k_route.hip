@@ -15,6 +15,7 @@
 #include "wave_ops.hpp"
 #include "launch.hpp"
 #include "q8h.hpp"
+#include "b32.hpp"
 
 namespace mimoe {
 
@@ -363,6 +364,22 @@ __device__ __forceinline__ void rt_transpose(const float4 (&in)[4], float4 *stag
     wave_lds_sync();   // the stage is rewritten next
 }
 
+// The operand rows that Q4_0 / Q5_0 / Q8_0 / F16 tables take (o.b32), of the
+// slab's tokens t0 .. t0 + 15: 8-value chunks dealt to the threads of the
+// slab's nwg work-groups, four threads per block.  As a launch of its own
+// (k_prep_b32) the pass takes 3.8 - 5 us, most of it beginning and end.  Layer us, so / in the
+// router's launch: moondream3 Q8_0 T = 5 70.5 / 69.1, T = 600 206.5 / 204.2,
+// diffusiongemma F16 T = 256 327.9 / 325.5, nemotronomni Q5_0 T = 200 331.5 /
+// 329.6.
+__device__ __forceinline__ void front_b32(const Q8Out &o, int64_t t0, int64_t T, int D, int wg, int nwg) {
+    const int nch = (int)((o.b32.mode == B32_PREP_CODES ? D : o.b32.ldo) / 8);   // a multiple of 4
+    const int rows = T - t0 < 16 ? (int)(T - t0) : 16, step = nwg * (int)blockDim.x;
+    for (int i = wg * (int)blockDim.x + (int)threadIdx.x; i < rows * nch; i += step) {
+        const int r = i / nch;
+        b32_prep8<true>(o.b_src + (t0 + r) * o.b_ld, t0 + r, i - r * nch, D, o.b32);
+    }
+}
+
 // The front of a forward: every work-group computes its logit tile, and with
 // a Q8_K output (o.q8 or o.xh set) quantizes its share of the slab's x rows
 // (row group item i = row * ngrp + grp by work-group i % net, wave i / net
@@ -412,7 +429,9 @@ __global__ void __launch_bounds__(1024) k_front(const float *__restrict__ W, con
         __syncthreads();   // the partials are rewritten next
         g0 = g1;
     }
-    if (o.q8 || o.xh) {
+    if constexpr (XO == XO_B32) {
+        front_b32(o, t0, T, D, et, net);
+    } else if (o.q8 || o.xh) {
         const int nb = D / QK, ngrp = (nb + 3) >> 2;
         for (int i = et + net * wave; i < 16 * ngrp; i += net * RT_WAVES) {
             const int64_t row = t0 + i / ngrp;
@@ -486,7 +505,9 @@ __global__ void __launch_bounds__(1024) k_front_parts(const float *__restrict__ 
             if (tt < T && ee < E) parts[((int64_t)c * T + tt) * E + ee] = part[r];
         }
     }
-    if (o.q8 || o.xh) {
+    if constexpr (XO == XO_B32) {
+        front_b32(o, t0, T, D, et * nsp + split, net * nsp);
+    } else if (o.q8 || o.xh) {
         const int nb = D / QK, ngrp = (nb + 3) >> 2;
         const int nwg = net * nsp, wg = et * nsp + split, nw = (int)(blockDim.x >> 6);
         for (int i = wg + nwg * wave; i < 16 * ngrp; i += nwg * nw) {
@@ -499,18 +520,29 @@ __global__ void __launch_bounds__(1024) k_front_parts(const float *__restrict__ 
     }
 }
 
+static bool front_vec(const float *W, const float *x, int64_t ldx, int D) {
+    return D % 64 == 0 && ldx % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)W % 16 == 0;
+}
+
+bool front_takes_b32(const float *W, const float *x, int64_t ldx, int D, const float *src, int64_t ld) {
+    return front_vec(W, x, ldx, D) && ld % 4 == 0 && (uintptr_t)src % 16 == 0 && D <= 65536;
+}
+
 int launch_front(const float *W, const float *b, const float *x, int64_t ldx, int64_t T, int D, int E,
                  float *logits, const Q8Out *qx, hipStream_t st) {
     if (T <= 0) return 0;
     const int nch = (D + 63) / 64;
     if (nch > RM_LIMIT_CHUNKS || T > (nch > RM_MAX_CHUNKS ? RM_LIMIT_WIDE_T : (int64_t)1 << 30)) return -6;
-    if (qx && D % QK) return -6;
-    const bool vec = (D % 64 == 0) && (ldx % 4 == 0) && ((uintptr_t)x % 16 == 0) && ((uintptr_t)W % 16 == 0);
+    const bool vec = front_vec(W, x, ldx, D), b32 = qx && qx->b_src;
+    if (qx && (b32 ? !front_takes_b32(W, x, ldx, D, qx->b_src, qx->b_ld) : D % QK != 0)) return -6;
     const int64_t net = (E + 15) / 16, nslab = (T + 15) / 16;
     const int64_t blocks = 8 * net * ((nslab + 7) / 8);
     if (blocks > 0x7fffffff) return -6;
     const Q8Out o = qx ? *qx : Q8Out{};
-    if (vec && q8_xo(o) == XO_Q4)
+    if (b32)
+        hipLaunchKernelGGL((k_front<true, XO_B32>), dim3((unsigned)blocks), dim3(64 * RT_WAVES), 0, st, W, b, x, ldx,
+                           T, D, E, logits, o);
+    else if (vec && q8_xo(o) == XO_Q4)
         hipLaunchKernelGGL((k_front<true, XO_Q4>), dim3((unsigned)blocks), dim3(64 * RT_WAVES), 0, st, W, b, x, ldx,
                            T, D, E, logits, o);
     else if (vec && q8_xo(o) == XO_Q6)
@@ -530,14 +562,16 @@ int launch_front_parts(const float *W, const float *x, int64_t ldx, int64_t T, i
     if (T <= 0) return 0;
     const int nch = (D + 63) / 64;
     if (nch > RM_LIMIT_CHUNKS || cps < 1 || cps > RT_WAVES || T > (int64_t)1 << 24) return -6;
-    if (qx && D % QK) return -6;
-    const bool vec = (D % 64 == 0) && (ldx % 4 == 0) && ((uintptr_t)x % 16 == 0) && ((uintptr_t)W % 16 == 0);
+    const bool vec = front_vec(W, x, ldx, D), b32 = qx && qx->b_src;
+    if (qx && (b32 ? !front_takes_b32(W, x, ldx, D, qx->b_src, qx->b_ld) : D % QK != 0)) return -6;
     const int64_t nsp = (nch + cps - 1) / cps, net = (E + 15) / 16, nslab = (T + 15) / 16;
     const int64_t blocks = nslab * net * nsp;
     if (blocks > 0x7fffffff) return -6;
     const Q8Out o = qx ? *qx : Q8Out{};
     const dim3 grid((unsigned)blocks), block((unsigned)(64 * cps));
-    if (vec && q8_xo(o) == XO_Q4)
+    if (b32)
+        hipLaunchKernelGGL((k_front_parts<true, XO_B32>), grid, block, 0, st, W, x, ldx, T, D, E, cps, parts, o);
+    else if (vec && q8_xo(o) == XO_Q4)
         hipLaunchKernelGGL((k_front_parts<true, XO_Q4>), grid, block, 0, st, W, x, ldx, T, D, E, cps, parts, o);
     else if (vec && q8_xo(o) == XO_Q6)
         hipLaunchKernelGGL((k_front_parts<true, XO_Q6>), grid, block, 0, st, W, x, ldx, T, D, E, cps, parts, o);

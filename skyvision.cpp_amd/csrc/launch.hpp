@@ -35,6 +35,17 @@ int launch_rmsnorm(const float *x, int64_t T, int D, float eps, float *y, hipStr
 // y = norm(x) per row of D <= 4096 (norm.hpp; x may equal y)
 int launch_norm(const NormParams &p, const float *x, int64_t T, int D, float *y, hipStream_t st);
 
+// the activation operands of one consumer weight type of the 32-value types and F16 (k_b32.hip)
+enum { B32_PREP_NONE = -1, B32_PREP_CODES = 0, B32_PREP_DQ = 1, B32_PREP_F16 = 2 };
+struct B32Prep {
+    int mode = B32_PREP_NONE;  // CODES: Q8_0 codes + scales (GEMV of Q4_0/Q5_0/Q8_0); DQ: fp16(d q) rows
+                               // (their GEMM); F16: fp16(x) rows (F16 tables, both paths)
+    int8_t *q8 = nullptr;      // CODES: [rows][K]
+    uint32_t *ds = nullptr;    // CODES: [rows][K/32] {fp16 scale bits, sum of the 32 codes << 16}
+    _Float16 *xh = nullptr;    // DQ / F16: [rows][ldo]
+    int64_t ldo = 0;           // >= K; values K .. ldo - 1 of a row are written as zeros
+};
+
 // ---- routing (k_route.hip)
 struct Q8Out {
     int8_t *q8 = nullptr;        // [rows][K] natural order (GEMV path)
@@ -47,7 +58,13 @@ struct Q8Out {
     _Float16 *xbs = nullptr;     // [rows][K/16] block sums of 16 codes, as fp16 (exact)
     int pre_act = 0;             // 4 (ACT_RELU_SQR): quantize relu(v)^2 instead of v
     int32_t *range_total = nullptr;   // [1] or null: blocks whose xh saturated at the fp16 range
+    // the router's launch only, in place of the above: rows b_src (b_ld apart)
+    // as b32 asks (where front_takes_b32)
+    B32Prep b32;
+    const float *b_src = nullptr;
+    int64_t b_ld = 0;
 };
+bool front_takes_b32(const float *W, const float *x, int64_t ldx, int D, const float *src, int64_t ld);
 // quantize rows of src (row r at src + r*ld values, fp32 or fp16) to Q8_K
 int launch_q8k_rows(const float *src, int64_t ld, int64_t nrows, int64_t K, const Q8Out &o, hipStream_t st);
 int launch_q8k_rows(const _Float16 *src, int64_t ld, int64_t nrows, int64_t K, const Q8Out &o, hipStream_t st);
@@ -251,16 +268,6 @@ int gemm_gs_wgs_per_cu(int glu);
 // weight rows of 32-value blocks (F16: 32 values per "block"), bit for bit the
 // CPU oracle's ggml _ref quantizers / fp16 rounding
 int launch_quantize_b32(int type, const float *src, void *dst, int64_t nblocks, hipStream_t st);
-// the activation operands of one consumer weight type
-enum { B32_PREP_CODES = 0, B32_PREP_DQ = 1, B32_PREP_F16 = 2 };
-struct B32Prep {
-    int mode;                  // CODES: Q8_0 codes + scales (GEMV of Q4_0/Q5_0/Q8_0); DQ: fp16(d q) rows
-                               // (their GEMM); F16: fp16(x) rows (F16 tables, both paths)
-    int8_t *q8 = nullptr;      // CODES: [rows][K]
-    uint32_t *ds = nullptr;    // CODES: [rows][K/32] {fp16 scale bits, sum of the 32 codes << 16}
-    _Float16 *xh = nullptr;    // DQ / F16: [rows][ldo]
-    int64_t ldo = 0;           // >= K; values K .. ldo - 1 of a row are written as zeros
-};
 int launch_prep_b32(const float *src, int64_t ld, int64_t nrows, int64_t K, const B32Prep &o, hipStream_t st);
 // Grouped GEMV.  Plain product: fp32 rows y.  glu / relu_sqr: the activation
 // rows leave as the next product's operand (rows of ncols values: fp16 oxh

@@ -22,7 +22,7 @@ namespace mimoe {
 
 // fp16 orders of Q8_K outputs: XO_Q4 / XO_Q6 the 32x32x16 order of a Q4_K /
 // Q6_K consumer, XO_ANY element by element (whatever the output asks for)
-enum { XO_ANY = 0, XO_Q4 = 1, XO_Q6 = 2 };
+enum { XO_ANY = 0, XO_Q4 = 1, XO_Q6 = 2, XO_B32 = 3 };
 
 // first of lane s's 4 values A of half g (B: the 4 at + 32); output slot p
 // = 0..7 of the half holds Q4_K A0 A2 B0 B2 A1 A3 B1 B3, Q6_K A0..A3 B0..B3

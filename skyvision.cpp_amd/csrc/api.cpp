@@ -7,8 +7,8 @@
 //   -> down -> weighted combine (+residual)
 // Decode-sized calls use the grouped integer-dot GEMV kernels, larger calls
 // the grouped MFMA GEMM kernels (use_gemm: by default from half a dispatched
-// row per expert on average for Q4_K / Q6_K tables, use_gemm_wide: from 1.25
-// for the others).
+// row per expert on average for Q4_K / Q6_K tables, use_gemm_b32: from 1.25 or
+// 1.5 for the others).
 // All workspace comes from mi_moe_ctx_reserve; forward calls never allocate.
 #include <hip/hip_runtime.h>
 
@@ -414,12 +414,24 @@ bool use_gemm(const mi_moe_ctx *c, int64_t T, int K, int E) {
     if (c->gemm_threshold > 0) return T >= c->gemm_threshold;
     return 2 * T * K >= (int64_t)E;
 }
-// The switch of the products still on 192-row tiles (mul_mat_id) and of
-// the Q4_0 / Q5_0 / Q8_0 / F16 tables, as measured on them: the GEMM above
-// 1.25 dispatched rows per expert.
+// The switch of mul_mat_id (192-row tiles): the GEMM above 1.25 dispatched
+// rows per expert.
 bool use_gemm_wide(const mi_moe_ctx *c, int64_t T, int K, int E) {
     if (c->gemm_threshold > 0) return T >= c->gemm_threshold;
     return 4 * T * K > 5 * (int64_t)E;
+}
+
+// The switch of the Q4_0 / Q5_0 / Q8_0 / F16 layers: the GEMM above 1.25
+// dispatched rows per expert, above 1.5 for Q8_0 and F16, whose GEMM has less
+// to gain (no nibbles to unpack once per row tile).  Layer us, GEMV / GEMM:
+// Q8_0 qwen3omni T = 24 (1.5 rows) 160.6 / 170.5, 32 (2) 186.6 / 189.7;
+// moondream3 12 (1.5) 112.7 / 124.5, 24 (3) 154.5 / 133.1; nemotronomni 32
+// (1.5) 300 / 299; F16 diffusiongemma 24 (1.5) 240 / 259, 32 (2) 276 / 273;
+// Q5_0 qwen3omni 20 (1.25) 133 / 145, 24 148 / 153, 32 175 / 159, nemotronomni
+// 24 (1.1) 235 / 227; Q4_0 moondream3 10 (1.25) 86.9 / 86.2, 16 110 / 96.
+bool use_gemm_b32(const mi_moe_ctx *c, int64_t T, int K, int E, int type) {
+    if (c->gemm_threshold > 0) return T >= c->gemm_threshold;
+    return type == MI_TYPE_Q8_0 || type == MI_TYPE_F16 ? 2 * T * K > 3 * (int64_t)E : 4 * T * K > 5 * (int64_t)E;
 }
 
 // the grouped MFMA GEMMs (else the grouped GEMV) for a k-quant layer
@@ -560,7 +572,7 @@ int64_t gb_max_tokens(int64_t halfs) { return GB_MAX_X / (2 * halfs); }
 bool gb_strides_ok(const mi_tensor &t) { return (int64_t)t.nb[1] <= GB_MAX_ROW_BYTES; }
 // the grouped GEMM for a routed call (row strides past its 32-bit offsets keep the GEMV)
 bool gb_path(const mi_moe_ctx *c, const mi_moe_layer *L, int64_t T) {
-    return use_gemm_wide(c, T, L->n_expert_used, L->n_expert) && gb_strides_ok(L->gate) && gb_strides_ok(L->down) &&
+    return use_gemm_b32(c, T, L->n_expert_used, L->n_expert, L->gate.type) && gb_strides_ok(L->gate) && gb_strides_ok(L->down) &&
            (!act_gated(L->act) || L->fused_gate_up || gb_strides_ok(L->up));
 }
 // The GEMV runs the shared expert's tokens four to a pass over its rows, one

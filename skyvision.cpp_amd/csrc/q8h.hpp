@@ -21,7 +21,8 @@
 namespace mimoe {
 
 // fp16 orders of Q8_K outputs: XO_Q4 / XO_Q6 the 32x32x16 order of a Q4_K /
-// Q6_K consumer, XO_ANY element by element (whatever the output asks for)
+// Q6_K consumer, XO_ANY element by element (whatever the output asks for),
+// XO_B32 the operand rows of the 32-value types and F16 instead (Q8Out::b32)
 enum { XO_ANY = 0, XO_Q4 = 1, XO_Q6 = 2, XO_B32 = 3 };
 
 // first of lane s's 4 values A of half g (B: the 4 at + 32); output slot p

@@ -270,7 +270,9 @@ int mi_norm(mi_moe_ctx *ctx, const mi_moe_norm *norm, const float *x, int64_t n_
  * w: F32 [T][K] device.  The layer's router and shared-expert fields are
  * ignored.  Ids must lie in [0, E): a slot whose gate/up or down id lies
  * outside contributes nothing to its token's sum (the other slots still do)
- * and is counted for mi_moe_ctx_take_errors. */
+ * and is counted for mi_moe_ctx_take_errors.  One or two tokens of a gated
+ * Q4_K layer run as one fused launch per token where out lies apart from the
+ * inputs (out == res is fine). */
 int mi_moe_expert_ffn(mi_moe_ctx *ctx, const mi_moe_layer *layer, const float *x, int64_t n_tokens,
                       const float *res, const int32_t *gate_up_ids, const int32_t *down_ids,
                       const float *w, float *out, mi_stream_t stream);

@@ -300,16 +300,16 @@ __device__ __forceinline__ void gv_pass(const B32Side &s, int kdiv, const uint8_
 //
 // What bounds it: the load path (a block is 2 - 3 loads of at most 16 bytes
 // at dword-aligned addresses; the same bytes at their own, 2-byte aligned
-// addresses: moondream3 Q8_0 T = 5 gate/up 36.7 against 31.2 us, down 24.5
+// addresses: qwen3omni Q8_0 T = 5 gate/up 36.7 against 31.2 us, down 24.5
 // against 19.8) and the work-groups in flight (four blocks ahead with one
 // token in the pass, two with more: at 125 registers 16 waves per CU; eight
 // ahead spills, 24 - 32 waves per CU with two tokens a pass are slower for
 // many rows).  Against the form before (each lane reading its blocks dword by
 // dword and the activations from the caches for every token anew, the GLU
 // rows quantized by a launch of their own, a dispatch launch, the shared
-// expert as a layer of its own), layer us: moondream3 Q8_0 T = 1 / 5 47.6 /
-// 78.5 -> 37 / 71, Q4_0 T = 5 72 -> 62; qwen3omni Q5_0 T = 12 127 -> 101,
-// Q8_0 T = 16 150 -> 131; nemotronomni Q5_0 T = 1 / 4 / 16 109 / 177 / 302 ->
+// expert as a layer of its own), layer us: moondream3 Q8_0 T = 1 47.6 -> 37,
+// Q4_0 T = 5 72 -> 62; qwen3omni Q8_0 T = 5 / 16 78.5 / 150 -> 71 / 131 (69
+// with x's codes from the router's launch), Q5_0 T = 12 127 -> 101; nemotronomni Q5_0 T = 1 / 4 / 16 109 / 177 / 302 ->
 // 47 / 80 / 176; diffusiongemma F16 T = 4 / 16 104 / 273 -> 95 / 203.
 enum { GV_STORE = 0, GV_GLU = 1, GV_RELU_SQR = 2 };
 template <int WT, int EPI, bool SH>

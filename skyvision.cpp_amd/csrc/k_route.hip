@@ -368,7 +368,7 @@ __device__ __forceinline__ void rt_transpose(const float4 (&in)[4], float4 *stag
 // slab's tokens t0 .. t0 + 15: 8-value chunks dealt to the threads of the
 // slab's nwg work-groups, four threads per block.  As a launch of its own
 // (k_prep_b32) the pass takes 3.8 - 5 us, most of it beginning and end.  Layer us, so / in the
-// router's launch: moondream3 Q8_0 T = 5 70.5 / 69.1, T = 600 206.5 / 204.2,
+// router's launch: qwen3omni Q8_0 T = 5 70.5 / 69.1, moondream3 T = 600 206.5 / 204.2,
 // diffusiongemma F16 T = 256 327.9 / 325.5, nemotronomni Q5_0 T = 200 331.5 /
 // 329.6.
 __device__ __forceinline__ void front_b32(const Q8Out &o, int64_t t0, int64_t T, int D, int wg, int nwg) {

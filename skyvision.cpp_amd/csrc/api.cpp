@@ -692,7 +692,7 @@ int run_experts_b32(mi_moe_ctx *c, const mi_moe_layer *L, const float *x, int64_
             g.q8 = ab.q8; g.ds = (const uint32_t *)ab.bs; g.xh = ab.h;
             g.counts = d.counts; g.offsets = d.offsets; g.perm = d.perm; g.active_e = d.active_e;
             g.n_active = d.n_active; g.max_active = max_active;
-            if (self_disp) { g.ids = ids_gu; g.rows = rows; }
+            if (self_disp) { g.ids = ids_gu; g.rows = rows; g.n_expert = E; }
             return g;
         };
         B32Args a = args_for(as_mat(L->gate), dg, c->ax, 1);
@@ -700,6 +700,7 @@ int run_experts_b32(mi_moe_ctx *c, const mi_moe_layer *L, const float *x, int64_
         a.glu = gated ? 1 : 0; a.relu_sqr = gated ? 0 : 1; a.fused = L->fused_gate_up;
         a.ncols = I; a.next_f16 = L->down.type == MI_TYPE_F16;
         a.oq8 = c->aact.q8; a.ods = (uint32_t *)c->aact.bs; a.oxh = c->aact.h;
+        a.bad_total = c->bad_total;   // (with ids: once per call, here)
         if (sh_here) {
             const int64_t S = L->sh_n_ff;
             a.sh_rows = T;

@@ -296,7 +296,7 @@ __device__ __forceinline__ void gv_pass(const B32Side &s, int kdiv, const uint8_
 // work-group's 32 columns are one Q8_0 block of each row), the bits of
 // launch_prep_b32 on the fp32 values.  With g.ids the expert list comes from
 // the ids: work-group row j belongs to slot j, and leaves unless the slot is
-// its expert's first.  SH: the shared expert's work-groups come first.
+// its expert's first (and its id one of the n_expert).  SH: the shared expert's work-groups come first.
 //
 // What bounds it: the load path (a block is 2 - 3 loads of at most 16 bytes
 // at dword-aligned addresses; the same bytes at their own, 2-byte aligned
@@ -335,6 +335,12 @@ __global__ void __launch_bounds__(64 * GV_WAVES) __attribute__((amdgpu_waves_per
         if (g.ids) {
             const int id = tid < g.rows ? g.ids[tid] : -1;
             e = g.ids[j];
+            // (before any address is formed from it; past here no thread
+            // without a slot matches e)
+            if ((unsigned)e >= (unsigned)g.n_expert) {
+                if (g.bad_total && cb == 0 && tid == 0) atomicAdd(g.bad_total, 1);
+                return;
+            }
             const uint64_t m = __ballot(id == e);
             if (lane == 0) s_cnt[wave] = __popcll(m);
             __syncthreads();
@@ -433,7 +439,7 @@ static int gv_launch(const B32Args &a, hipStream_t st) {
 int launch_gemv_b32(const B32Args &g, hipStream_t st) {
     if (g.max_active <= 0) return 0;
     if (g.a.K % 32 || g.a.K > 0x7fffffff) return -6;
-    if (g.ids && g.rows > GV_SD_IDS) return -6;
+    if (g.ids && (g.rows > GV_SD_IDS || g.n_expert <= 0)) return -6;
     if ((g.glu || g.relu_sqr) && g.ncols % 32) return -6;
     if (g.sh_rows > 0 && (g.sh.a.type != g.a.type || g.sh.a.K % 32 || ((g.glu || g.relu_sqr) && g.sh.ncols % 32))) return -6;
 #define GV_TYPE(T)                                                \

@@ -273,7 +273,9 @@ int launch_prep_b32(const float *src, int64_t ld, int64_t nrows, int64_t K, cons
 // rows leave as the next product's operand (rows of ncols values: fp16 oxh
 // with next_f16, else codes oq8 and words ods; ncols % 32 == 0).  ids: the
 // rows' expert ids, at most GV_SD_IDS of them, in place of the dispatch's
-// lists.  A shared expert (sh_rows > 0) as in GBArgs.
+// lists; a row whose id lies outside [0, n_expert) is not computed, its output
+// row is not written, and it is counted in bad_total (NULL: not counted), as
+// by the dispatch.  A shared expert (sh_rows > 0) as in GBArgs.
 struct B32Side {
     ExpertMat a, b;            // b: up table (separate gate/up GLU), else unused
     int fused;
@@ -296,6 +298,8 @@ struct B32Args : B32Side {
     int max_active;
     const int32_t *ids;
     int64_t rows;
+    int n_expert;              // with ids
+    int32_t *bad_total;
     B32Side sh;
     int64_t sh_rows;
     const float *sh_w;

@@ -235,6 +235,10 @@ __device__ inline float softmax_selected_wave(float myval, int K, int lane) {
 // wave's largest remaining value (a max reduction), whose id is the lowest
 // set bit of a ballot of its holders (ids 64 i + lane, block i = 0 first);
 // the winner then leaves the race (NaN: the max skips it, == never holds).
+// Once no number is left among a token's values (a NaN or an infinity in its
+// row), the remaining slots take the lowest ids not taken yet with the value
+// NaN: ids stay in [0, E) and distinct, and the token's weights are NaN (kind
+// 1 below weighs by the slots' own logits).
 // The order equals ranking every value by the values that come before it
 // (larger, or equal with a lower id).  Lane k < K gets the k-th id and, when
 // want_w, its softmax weight over the K selected logits: max, expf(v - max),
@@ -323,7 +327,7 @@ __device__ inline void topk_softmax_regs(const float (&raw)[TOPK_MAX_PER_LANE], 
 #pragma unroll
         for (int i = 1; i < TOPK_MAX_PER_LANE; ++i)
             if (i < nper) m = fmaxf(m, v[i]);
-        const float s = wave_max_uniform(m);
+        float s = wave_max_uniform(m);
         int e = -1;
 #pragma unroll
         for (int i = 0; i < TOPK_MAX_PER_LANE; ++i) {
@@ -332,6 +336,11 @@ __device__ inline void topk_softmax_regs(const float (&raw)[TOPK_MAX_PER_LANE], 
             if (e < 0 && b != 0ull) e = 64 * i + (int)__builtin_ctzll(b);
         }
         e = __builtin_amdgcn_readfirstlane(e);
+        if ((unsigned)e >= (unsigned)E) {   // nothing equals NaN; the lanes past E hold -inf
+            e = 0;
+            while (__ballot(lane < r && mysel == e)) ++e;   // (r < K <= E ids are taken)
+            s = __builtin_nanf("");
+        }
 #pragma unroll
         for (int i = 0; i < TOPK_MAX_PER_LANE; ++i)
             if (e == 64 * i + lane) v[i] = __builtin_nanf("");

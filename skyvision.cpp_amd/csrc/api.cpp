@@ -569,11 +569,15 @@ int gb_bm(const mi_moe_ctx *c, int64_t rows, int E, int64_t ncols) {
 // tokens per pass of a call whose rows hold at most `halfs` fp16 values per
 // token (larger calls run in passes)
 int64_t gb_max_tokens(int64_t halfs) { return GB_MAX_X / (2 * halfs); }
+int64_t gb_layer_tokens(const mi_moe_layer *L) {
+    return gb_max_tokens(std::max(round_up(L->n_embd, 64), L->n_expert_used * round_up(L->n_ff, 64)));
+}
 bool gb_strides_ok(const mi_tensor &t) { return (int64_t)t.nb[1] <= GB_MAX_ROW_BYTES; }
-// the grouped GEMM for a routed call (row strides past its 32-bit offsets keep the GEMV)
+// the grouped GEMM for a routed call (row strides, or a single token's rows,
+// past its 32-bit offsets keep the GEMV)
 bool gb_path(const mi_moe_ctx *c, const mi_moe_layer *L, int64_t T) {
     return use_gemm_b32(c, T, L->n_expert_used, L->n_expert, L->gate.type) && gb_strides_ok(L->gate) && gb_strides_ok(L->down) &&
-           (!act_gated(L->act) || L->fused_gate_up || gb_strides_ok(L->up));
+           (!act_gated(L->act) || L->fused_gate_up || gb_strides_ok(L->up)) && gb_layer_tokens(L) > 0;
 }
 // The GEMV runs the shared expert's tokens four to a pass over its rows, one
 // pass after another, beside the routed experts' work-groups: up to this many
@@ -591,8 +595,7 @@ bool b32_shared_ok(const mi_moe_ctx *c, const mi_moe_layer *L, int64_t T) {
     if (!gb_path(c, L, T)) return T <= GV_SHARED_T;
     if (!gb_strides_ok(L->sh_gate) || !gb_strides_ok(L->sh_down) || (act_gated(L->act) && !gb_strides_ok(L->sh_up)))
         return false;
-    const int64_t K = L->n_expert_used;
-    return T <= gb_max_tokens(std::max({round_up(L->n_embd, 64), K * round_up(L->n_ff, 64), round_up(L->sh_n_ff, 64)}));
+    return T <= std::min(gb_layer_tokens(L), gb_max_tokens(round_up(L->sh_n_ff, 64)));
 }
 
 // the operand form of x for the gate/up product
@@ -624,7 +627,7 @@ int run_experts_b32(mi_moe_ctx *c, const mi_moe_layer *L, const float *x, int64_
     const bool gated = act_gated(L->act);
     const bool gemm = gb_path(c, L, T);
     const int64_t ldx = round_up(D, 64), ldi = round_up(I, 64);
-    const int64_t tmax = gb_max_tokens(std::max(ldx, K * ldi));
+    const int64_t tmax = gb_layer_tokens(L);
     if (gemm && T > tmax) {
         // in passes; then the dispatch of the whole call, whose counts, offsets and lists the caller may read
         for (int64_t t0 = 0; t0 < T; t0 += tmax) {
@@ -1329,7 +1332,7 @@ int forward_impl(mi_moe_ctx *c, const mi_moe_layer *L, const float *x, int64_t T
         bool xq = !xr && x_q8_spec(c, L, T, qx);
         const float *xrow = xr ? xr : x;
         if (is_b32f(L->gate.type) && front_takes_b32(L->router_w, xrow, D, D, x, D) &&
-            (!gb_path(c, L, T) || T <= gb_max_tokens(std::max(round_up(D, 64), K * round_up(L->n_ff, 64))))) {
+            (!gb_path(c, L, T) || T <= gb_layer_tokens(L))) {
             qx = Q8Out{};
             qx.b32 = b32_x_prep(c, L, T);
             qx.b_src = x;
@@ -1567,9 +1570,10 @@ int mi_mul_mat_id(mi_moe_ctx *c, const mi_tensor *as, const mi_tensor *b, const 
     HIP_TRY(hipSetDevice(c->device));
     hipStream_t st = (hipStream_t)stream;
     const int64_t rows = T * n_used;
-    // the grouped GEMM of the 32-value types and F16, in passes past its 32-bit offsets
-    const bool gb = is_b32f(as->type) && use_gemm_wide(c, T, (int)n_used, (int)E) && gb_strides_ok(*as);
+    // the grouped GEMM of the 32-value types and F16, in passes past its 32-bit
+    // offsets (a single token's rows past them: the GEMV)
     const int64_t ldx = round_up(Kin, 64), tmax = gb_max_tokens(ne11 * ldx);
+    const bool gb = is_b32f(as->type) && use_gemm_wide(c, T, (int)n_used, (int)E) && gb_strides_ok(*as) && tmax > 0;
     if (gb && T > tmax) {
         for (int64_t t0 = 0; t0 < T; t0 += tmax) {
             const int64_t n = std::min(tmax, T - t0);

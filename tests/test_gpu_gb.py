@@ -164,3 +164,27 @@ def test_more_rows_than_one_pass_holds():
         assert np.array_equal(small.download(np.uint32, (n, D)), out.download(np.uint32, (n, D), 4 * lo * D))
     assert ctx.take_errors() == (0, 0)
     ctx.close()
+
+
+@pytest.mark.parametrize("T,n_used", [(1, 1_000_000), (2, 500_000)], ids=["one_token", "two_passes"])
+def test_mul_mat_id_rows_past_the_offsets(T, n_used):
+    """a token's rows past the GEMM's 32-bit buffer offsets (2.05e9 values: the
+    GEMV takes the call), and two tokens that fit only one by one (a pass
+    each): rows at both ends and on both sides of the seam against the oracle"""
+    t, Kin, N, E = M.TYPE_Q8_0, 2048, 32, 4
+    rng = np.random.default_rng(T)
+    wq = _quant(t, (rng.standard_normal((E, N, Kin)) * 0.05).astype(np.float32))
+    rows = T * n_used
+    ids = rng.integers(0, E, (T, n_used)).astype(np.int32)
+    ctx = M.Context(0)
+    ctx.reserve(rows, Kin, N, E, 1)
+    wd, b, idd, dst = M.to_device(wq), M.DeviceBuffer(4 * rows * Kin), M.to_device(ids), M.DeviceBuffer(4 * rows * N)
+    M.check("fill", ctx.fill_normal(b, rows * Kin, 7, 1, 0.0, 1.0))
+    M.check("mul_mat_id", ctx.mul_mat_id(M.tensor(wd, t, [Kin, N, E]), M.tensor(b, M.TYPE_F32, [Kin, n_used, T]),
+                                         M.tensor(idd, M.TYPE_I32, [n_used, T]), M.tensor(dst, M.TYPE_F32, [N, n_used, T])))
+    for lo in (0, rows // 2 - 30, rows - 60):
+        part = b.download(np.float32, (1, 60, Kin), 4 * lo * Kin)
+        ref = O.mul_mat_id(t, wq.reshape(E * N, -1), Kin, N, E, part, ids.ravel()[lo:lo + 60].reshape(1, -1))
+        assert rel_l2(dst.download(np.float32, (1, 60, N), 4 * lo * N), ref) <= (1e-4 if T == 1 else TOL[t])
+    assert ctx.take_errors() == (0, 0)
+    ctx.close()

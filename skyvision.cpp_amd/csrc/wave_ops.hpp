@@ -327,7 +327,7 @@ __device__ inline void topk_softmax_regs(const float (&raw)[TOPK_MAX_PER_LANE], 
 #pragma unroll
         for (int i = 1; i < TOPK_MAX_PER_LANE; ++i)
             if (i < nper) m = fmaxf(m, v[i]);
-        float s = wave_max_uniform(m);
+        const float s = wave_max_uniform(m);
         int e = -1;
 #pragma unroll
         for (int i = 0; i < TOPK_MAX_PER_LANE; ++i) {
@@ -336,17 +336,25 @@ __device__ inline void topk_softmax_regs(const float (&raw)[TOPK_MAX_PER_LANE], 
             if (e < 0 && b != 0ull) e = 64 * i + (int)__builtin_ctzll(b);
         }
         e = __builtin_amdgcn_readfirstlane(e);
-        if ((unsigned)e >= (unsigned)E) {   // nothing equals NaN; the lanes past E hold -inf
-            e = 0;
-            while (__ballot(lane < r && mysel == e)) ++e;   // (r < K <= E ids are taken)
-            s = __builtin_nanf("");
-        }
 #pragma unroll
         for (int i = 0; i < TOPK_MAX_PER_LANE; ++i)
             if (e == 64 * i + lane) v[i] = __builtin_nanf("");
         if (lane == r) {
             mysel = e;
             mys = s;
+        }
+    }
+    // the slots past the numbers: -1 (nothing equals NaN) or a lane past E
+    // (-inf); the last ones, r0 .. K - 1
+    const uint64_t none = __ballot(lane < K && (unsigned)mysel >= (unsigned)E);
+    if (none) {
+        for (int r = (int)__builtin_ctzll(none); r < K; ++r) {
+            int e = 0;
+            while (__ballot(lane < r && mysel == e)) ++e;   // (r < K <= E ids are taken)
+            if (lane == r) {
+                mysel = e;
+                mys = __builtin_nanf("");
+            }
         }
     }
     if (!want_w) {

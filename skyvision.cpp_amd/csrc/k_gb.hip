@@ -307,6 +307,11 @@ __device__ __forceinline__ void gb_kloop(rsrc_t rx, const uint32_t *aoff, const 
         __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): the blocks are in registers
         const bool second = full || kb + KA < nk, next = full || st + 1 < nst;
         if (second) issue_a(kb + KA, a1);
+        // The counted wait in front of the second half (2 NLD loads may stay
+        // out) holds only if these activation loads go out before all of the
+        // weight loads: no pass of the compiler may exchange them (the two go
+        // to different LDS arrays, so nothing else orders them).
+        asm volatile("" ::: "memory");
         if (next) {
 #pragma unroll
             for (int ct = 0; ct < 2; ++ct) wd[ct].issue(ws + (wbase + ct * gb_wtile<WT, KG>()), st + 1);

@@ -1593,12 +1593,13 @@ int decode1_max_grid(int device, int *grid) {
     if (e != hipSuccess) return record_hip_error(e);
     int per = 1;
     for (int dt = 12; dt <= 14; dt += 2)
-        for (int nbi = 1; nbi <= 8; ++nbi) {
-            int p = 0;
-            e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&p, decode1_fn(dt, false, nbi), DEC_THREADS, 0);
-            if (e != hipSuccess) return record_hip_error(e);
-            per = imin(per, p);
-        }
+        for (int ids = 0; ids < 2; ++ids)   // (both forms of the kernel)
+            for (int nbi = 1; nbi <= 8; ++nbi) {
+                int p = 0;
+                e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&p, decode1_fn(dt, ids != 0, nbi), DEC_THREADS, 0);
+                if (e != hipSuccess) return record_hip_error(e);
+                per = imin(per, p);
+            }
     *grid = cus * per;   // one WG per CU
     if (*grid > DEC_MAX_GRID) *grid = 0;
     return 0;

@@ -395,7 +395,7 @@ int mi_moe_ctx_stage_clock(mi_moe_ctx *ctx, const char *stage, double *ghz, int 
  * per expert); for Q4_0 / Q5_0 / Q8_0 / F16 tables and mi_moe_mul_mat_id
  * when 4 * T * K > 5 * E (more than 1.25 rows per expert). */
 int mi_moe_ctx_set_gemm_threshold(mi_moe_ctx *ctx, int64_t min_tokens_for_gemm);
-/* Row tiles of the grouped GEMMs of Q4_K gate/up layers: 0 (the default) by
+/* Row tiles of the grouped GEMMs.  Of Q4_K gate/up layers: 0 (the default) by
  * shape, 32-row tiles when the call dispatches at most 8 rows per expert on
  * average (qwen3omni up to 128 tokens, moondream3 up to 64: several
  * work-groups per CU keep more of the weight stream in flight), and within
@@ -409,10 +409,12 @@ int mi_moe_ctx_set_gemm_threshold(mi_moe_ctx *ctx, int64_t min_tokens_for_gemm);
  * ahead) on layers whose tables are all Q4_K with n_embd and n_ff <= 2048
  * (others take the shape rule); 4 8-row tiles wherever they apply (else
  * 32-row); 5 64-row tiles at every size.  Q6_K gate/up layers have the 32-
- * and 192-row tiles (kinds 2 and 4: 32-row; 1 and 5: 192-row).  Kinds 0-2, 4
- * and 5 give the same bits (the same per-row arithmetic); the skinny products sum each output's products in another
- * order (fp32; the rows agree to ~2e-4 rel-L2 after the activations' fp16
- * and Q8_K roundings). */
+ * and 192-row tiles (kinds 2 and 4: 32-row; 1 and 5: 192-row).  Q4_0 / Q5_0 / Q8_0
+ * / F16 layers and mi_mul_mat_id of such tables have 32- and 128-row tiles
+ * (kind 2: 32-row, 1: 128-row; others: by shape).  Kinds 0-2, 4 and 5 give the
+ * same bits (the same per-row arithmetic); the skinny products sum each
+ * output's products in another order (fp32; the rows agree to ~2e-4 rel-L2
+ * after the activations' fp16 and Q8_K roundings). */
 int mi_moe_ctx_set_gemm_tiles(mi_moe_ctx *ctx, int kind);
 /* Schedule of decode calls of mi_moe_forward (1 token, and batches of 2..16
  * tokens; for experts of more than 2 MiB, batches that dispatch at most one

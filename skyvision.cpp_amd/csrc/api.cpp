@@ -111,7 +111,9 @@ struct mi_moe_ctx {
     int32_t *bad_total = nullptr;   // caller ids outside [0, E) since the last take
     int32_t *range_total = nullptr; // GEMM-path Q8_K blocks saturated at the fp16 range
     int64_t gemm_threshold = 0;   // 0: the shape rule of use_gemm
-    int gemm_tiles = 0;           // Q4_K GEMM row tiles: 0 by shape, 1 G4_BM, 2 G4_BM_SMALL, 3 GS_BM (k_gs), 4 G4_BM_TINY, 5 G4_BM_MID
+    // k-quant GEMM row tiles: 0 by shape, 1 G4_BM, 2 G4_BM_SMALL, 3 GS_BM (k_gs), 4 G4_BM_TINY, 5 G4_BM_MID;
+    // 32-value types and F16: 1 GB_BM_LARGE, 2 GB_BM_SMALL, else by shape
+    int gemm_tiles = 0;
     int n_cu = 0;                 // compute units of the device
     // single-token fused kernel (k_decode.hip)
     int fused_decode = MI_DECODE_FUSED;
@@ -560,8 +562,10 @@ int64_t round_up(int64_t n, int64_t to) { return (n + to - 1) / to * to; }
 // box, 32 / 64 / 128-row tiles: qwen3omni T = 100 (6 rows per expert) 206 /
 // 222 / 207, T = 300 (19) 252 / 241 / 222, T = 600 (38) 332 / 275 / 253;
 // moondream3 T = 160 (20) 188 / 175 / 161.  A call of few work-groups (a
-// shared expert) keeps the small tiles, which are four times as many.
+// shared expert) keeps the small tiles, which are four times as many.  Kinds 1
+// and 2 of mi_moe_ctx_set_gemm_tiles ask for one or the other.
 int gb_bm(const mi_moe_ctx *c, int64_t rows, int E, int64_t ncols) {
+    if (c->gemm_tiles == 1 || c->gemm_tiles == 2) return c->gemm_tiles == 1 ? GB_BM_LARGE : GB_BM_SMALL;
     const int64_t wgs = (rows / GB_BM_LARGE + E) * (ncols / 256);
     return rows > 16 * (int64_t)E && wgs >= c->n_cu ? GB_BM_LARGE : GB_BM_SMALL;
 }

@@ -5,7 +5,8 @@ count of 32-value blocks (a half group at the end of a row) and widths no
 multiple of a work-group's columns, rows that start at a misaligned even byte
 (shifted tables, padded row strides), fused and separate gate/up, relu^2
 experts, down tables of another type than gate/up; and mul_mat_id with ids
-outside [0, E).
+outside [0, E).  Every case runs on the 32- and on the 128-row tiles, bit for
+bit the same.
 
 Bars: the quantized types 1e-2 against the oracle (fp16 operands: 2^-11 per
 weight and per activation, and one step of a Q8_0 code, 1 / 127 of a block's
@@ -74,10 +75,13 @@ def _run(t, td, D, I, E, K, counts, fused, act, pad=0, shift=0, seed=0):
              gating=M.GATING_SOFTMAX_TOPK)
     ref, _ = O.moe_forward(o, x, None, sel_in=ids, w_in=w)
     got = {}
-    for name, thr in (("gemm", 1), ("gemv", 1 << 30)):
+    for name, thr, kind in (("gemm", 1, 2), ("gemm128", 1, 1), ("gemm shape", 1, 0), ("gemv", 1 << 30, 0)):
         ctx.set_gemm_threshold(thr)
+        ctx.set_gemm_tiles(kind)
         M.check("expert_ffn", ctx.expert_ffn(L, xd, T, None, idd, idd, wd, out))
         got[name] = out.download(np.float32, (T, D))
+    for name in ("gemm128", "gemm shape"):   # both tile sizes: the same sums in the same order
+        assert np.array_equal(got[name].view(np.uint32), got["gemm"].view(np.uint32)), name
     assert ctx.take_errors() == (0, 0)
     ctx.close()
     e, ev = rel_l2(got["gemm"], ref), rel_l2(got["gemv"], ref)
@@ -125,13 +129,16 @@ def test_mul_mat_id_bad_ids(t):
     ctx = M.Context(0)
     ctx.reserve(T, Kin, Kin, E, n_used)
     bd, idd, dst = M.to_device(b), M.to_device(bad), M.DeviceBuffer(4 * T * n_used * N)
-    M.check("mul_mat_id", ctx.mul_mat_id(M.tensor(M.to_device(wq), t, [Kin, N, E]), M.tensor(bd, M.TYPE_F32, [Kin, n_used, T]),
-                                         M.tensor(idd, M.TYPE_I32, [n_used, T]), M.tensor(dst, M.TYPE_F32, [N, n_used, T])))
-    got = dst.download(np.float32, (T, n_used, N))
+    wd = M.to_device(wq)
     ref = O.mul_mat_id(t, wq.reshape(E * N, -1), Kin, N, E, b, ids)
     ref[bad != ids] = 0.0
-    assert not got[bad != ids].any() and rel_l2(got, ref) <= TOL[t]
-    assert ctx.take_errors()[0] == 2
+    for kind in (2, 1):
+        ctx.set_gemm_tiles(kind)
+        M.check("mul_mat_id", ctx.mul_mat_id(M.tensor(wd, t, [Kin, N, E]), M.tensor(bd, M.TYPE_F32, [Kin, n_used, T]),
+                                             M.tensor(idd, M.TYPE_I32, [n_used, T]), M.tensor(dst, M.TYPE_F32, [N, n_used, T])))
+        got = dst.download(np.float32, (T, n_used, N))
+        assert not got[bad != ids].any() and rel_l2(got, ref) <= TOL[t]
+        assert ctx.take_errors()[0] == 2
     ctx.close()
 
 

@@ -4,9 +4,9 @@ and the shared expert as a one-expert layer on mi_moe_expert_ffn (which runs
 the same arithmetic in launches of its own).  Both are fp32 values the forward
 adds once, so the sum is bit for bit; with a scalar gate row the weight is an
 fp32 sigmoid, computed here in fp64: two ulp of the weight times the value.
-Token counts around the 32- and 128-row tiles, shared widths with an odd
-number of blocks and more than a work-group's columns, tables the launch
-cannot share (another type, another activation) beside those it can.
+Token counts around the 32- and 128-row tiles, each run on both; shared widths
+with an odd number of blocks and more than a work-group's columns, tables the
+launch cannot share (another type, another activation) beside those it can.
 """
 import ctypes as C
 
@@ -89,6 +89,10 @@ def test_shared_in_the_routed_launches(T, sh_I, case, gated_row):
     shared = get()
     M.check("forward", ctx.forward(with_sh, xd, T, None, out))
     got = get()
+    for kind in (1, 2):   # 128- and 32-row tiles throughout
+        ctx.set_gemm_tiles(kind)
+        M.check("forward", ctx.forward(with_sh, xd, T, None, out))
+        assert np.array_equal(get().view(np.uint32), got.view(np.uint32)), kind
     assert ctx.take_errors() == (0, 0)
     ctx.close()
     want = routed + shared

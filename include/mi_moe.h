@@ -411,7 +411,8 @@ int mi_moe_ctx_set_gemm_threshold(mi_moe_ctx *ctx, int64_t min_tokens_for_gemm);
  * 32-row); 5 64-row tiles at every size.  Q6_K gate/up layers have the 32-
  * and 192-row tiles (kinds 2 and 4: 32-row; 1 and 5: 192-row).  Q4_0 / Q5_0 / Q8_0
  * / F16 layers and mi_mul_mat_id of such tables have 32- and 128-row tiles
- * (kind 2: 32-row, 1: 128-row; others: by shape).  Kinds 0-2, 4 and 5 give the
+ * (kind 2: 32-row, 1: 128-row; others: by shape), mi_mul_mat_id of F16 tables
+ * also 192-row tiles (kind 5; by shape above 32 rows per expert).  Kinds 0-2, 4 and 5 give the
  * same bits (the same per-row arithmetic); the skinny products sum each
  * output's products in another order (fp32; the rows agree to ~2e-4 rel-L2
  * after the activations' fp16 and Q8_K roundings). */

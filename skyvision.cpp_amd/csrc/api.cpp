@@ -112,7 +112,7 @@ struct mi_moe_ctx {
     int32_t *range_total = nullptr; // GEMM-path Q8_K blocks saturated at the fp16 range
     int64_t gemm_threshold = 0;   // 0: the shape rule of use_gemm
     // k-quant GEMM row tiles: 0 by shape, 1 G4_BM, 2 G4_BM_SMALL, 3 GS_BM (k_gs), 4 G4_BM_TINY, 5 G4_BM_MID;
-    // 32-value types and F16: 1 GB_BM_LARGE, 2 GB_BM_SMALL, else by shape
+    // 32-value types and F16: 1 GB_BM_LARGE, 2 GB_BM_SMALL, else by shape (5: GF_BM for mul_mat_id of F16)
     int gemm_tiles = 0;
     int n_cu = 0;                 // compute units of the device
     // single-token fused kernel (k_decode.hip)
@@ -568,6 +568,22 @@ int gb_bm(const mi_moe_ctx *c, int64_t rows, int E, int64_t ncols) {
     if (c->gemm_tiles == 1 || c->gemm_tiles == 2) return c->gemm_tiles == 1 ? GB_BM_LARGE : GB_BM_SMALL;
     const int64_t wgs = (rows / GB_BM_LARGE + E) * (ncols / 256);
     return rows > 16 * (int64_t)E && wgs >= c->n_cu ? GB_BM_LARGE : GB_BM_SMALL;
+}
+// mul_mat_id of F16 tables on the 192-row tiles of k_gf, against the 128-row
+// ones that it would take.  Call us, 128 / 192: K 1024, N 2048, E 64 at 25 rows
+// per expert 72.5 / 73.0, 38 79.0 / 76.5, 100 104 / 94, 125 130 / 98, 500 361 /
+// 265; K 704, N 2816, E 128 at 25 149 / 145, 38 166 / 154, 125 267 / 200; K
+// 1408, N 2048 at 50 104 / 106, 62 109 / 107, 125 154 / 125.  K 2048, N 2048 at
+// 62 161 / 162, 112 211 / 179; K 2048, N 768 at 125 194 / 172, but 188 (half of
+// the experts past one tile) 197 / 218.  K 2816, N 704: at 125 220 / 210, else
+// the 128-row tiles by 10 - 25 %.
+bool gf_tiles(const mi_moe_ctx *c, int type, int64_t rows, int E, int64_t K, int64_t N) {
+    if (type != MI_TYPE_F16 || rows / GF_BM + 1 + E > 65535) return false;   // (tiles: a grid dimension)
+    if (c->gemm_tiles == 1 || c->gemm_tiles == 2) return false;
+    if (c->gemm_tiles == 5) return true;
+    if ((rows / GF_BM + E) * (N / 128) < c->n_cu) return false;
+    if (K <= 1536) return rows > (K <= 1024 ? 32 : 56) * (int64_t)E;
+    return K <= 2048 && rows > 96 * (int64_t)E && (rows <= 160 * (int64_t)E || rows > 208 * (int64_t)E);
 }
 // the grouped GEMM reads its activation rows through 32-bit buffer offsets:
 // tokens per pass of a call whose rows hold at most `halfs` fp16 values per
@@ -1590,7 +1606,7 @@ int mi_mul_mat_id(mi_moe_ctx *c, const mi_tensor *as, const mi_tensor *b, const 
         return MI_MOE_OK;
     }
     const int max_active = (int)std::min<int64_t>(E, rows);
-    const int bm = gb ? gb_bm(c, rows, (int)E, N) : G4_BM;
+    const int bm = !gb ? G4_BM : gf_tiles(c, as->type, rows, (int)E, Kin, N) ? GF_BM : gb_bm(c, rows, (int)E, N);
     const int max_tiles = (int)((rows + bm - 1) / bm + max_active);
     const DispBuf &dsp = c->disp[0];
     Dispatch dv = dsp.view();

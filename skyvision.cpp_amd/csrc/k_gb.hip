@@ -489,6 +489,105 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
 #endif
 }
 
+// Plain product of F16 tables in tiles of at most GF_BM = 192 rows, for
+// mul_mat_id (the rule and its times: gf_tiles in api.cpp): 128 weight rows
+// per work-group, 32 per wave, each lane loading its own 16 bytes per step
+// (F16 needs no unpacking, so little is won by staging it), the next group
+// while the current one is computed; activations through 2 x 24 KB of LDS.
+// Three work-groups fit a CU, so one's start and stores run beside another's
+// K loop, which decides for a short K and many rows (k_gb with F16 has LDS for
+// one), and an expert of 129 - 192 rows is one tile.  The operands and their
+// order, and so the bits, are k_gb's.  K 1024, N 2048, E 64, 8000 rows: 130 us
+// in 128-row tiles of k_gb, 98 here (the call; 268 MB of weights).
+__global__ void __launch_bounds__(256) k_gf(GBArgs g) {
+    __shared__ __attribute__((aligned(16))) _Float16 As[2][GF_BM * 64];
+    __shared__ int s_row[GF_BM], s_p[GF_BM];   // activation and output row of each tile row (past the tile: row 0)
+    const int tile = blockIdx.y;
+    if (tile >= *g.n_tiles) return;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
+    const int e = g.tile_e[tile], start = g.tile_start[tile], mrows = g.tile_rows[tile];
+    const int nrt = (mrows + 31) >> 5;
+    const int64_t col = (int64_t)blockIdx.x * 128 + 32 * wave + l32, K = g.a.K;
+    const bool col_ok = col < g.ncols;
+    // (a column past the matrix: row 0, not stored)
+    const uint8_t *row = g.a.data + (int64_t)e * g.a.mat_bytes + (col_ok ? col : 0) * g.a.row_bytes;
+    if (tid < GF_BM) {
+        const int p = tid < mrows ? g.perm[start + tid] : -1;
+        s_p[tid] = p;
+        s_row[tid] = p < 0 ? 0 : (g.ne11 == 1 ? p / g.K : p);
+    }
+    __syncthreads();
+    // 16-byte piece q = tid + 256 i of a group: tile row q / 8, K chunk q % 8, in slot chunk ^ (row & 7)
+    constexpr int NC = GF_BM * 8 / 256;
+    uint4 areg[NC];
+    auto load_a = [&](int kb) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < NC; ++i) {
+            const int q = tid + 256 * i, r = q >> 3, c = q & 7;
+            areg[i] = r < 32 * nrt ? *(const uint4 *)(g.xh + (int64_t)s_row[r] * g.ldx + 64 * (int64_t)kb + 8 * c)
+                                   : make_uint4(0, 0, 0, 0);
+        }
+    };
+    auto store_a = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < NC; ++i) {
+            const int q = tid + 256 * i, r = q >> 3, c = q & 7;
+            *(uint4 *)(&As[buf][(r * 8 + (c ^ (r & 7))) * 8]) = areg[i];
+        }
+    };
+    // steps 0 - 3 of a group: values 8 s .. 8 s + 7 of block h (K % 64 = 32: zeros past the row)
+    auto load_w = [&](int kb, uint4 (&w)[4]) __attribute__((always_inline)) {
+        const int64_t k = 64 * (int64_t)kb + 32 * h;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) w[s] = k < K ? *(const uint4 *)(row + 2 * (k + 8 * s)) : make_uint4(0, 0, 0, 0);
+    };
+    f32x16 acc[GF_BM / 32];
+#pragma unroll
+    for (int t = 0; t < GF_BM / 32; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[t][i] = 0.f;
+    const int nk = (int)((K + 63) / 64);
+    uint4 cur[4], nxt[4];
+    load_a(0);
+    load_w(0, cur);
+    store_a(0);
+    __syncthreads();
+    for (int kb = 0; kb < nk; ++kb) {
+        const bool more = kb + 1 < nk;
+        if (more) {
+            load_a(kb + 1);
+            load_w(kb + 1, nxt);
+        }
+        const _Float16 *A = As[kb & 1];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const half8_t b = __builtin_bit_cast(half8_t, cur[s]);
+#pragma unroll
+            for (int t = 0; t < GF_BM / 32; ++t)
+                if (t < nrt) {
+                    const int r = 32 * t + l32;
+                    const half8_t a = *(const half8_t *)(&A[(r * 8 + ((4 * h + s) ^ (r & 7))) * 8]);
+                    acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, acc[t], 0, 0, 0);
+                }
+        }
+        if (more) {
+            store_a((kb + 1) & 1);
+#pragma unroll
+            for (int s = 0; s < 4; ++s) cur[s] = nxt[s];
+        }
+        __syncthreads();
+    }
+    if (!col_ok) return;
+#pragma unroll
+    for (int t = 0; t < GF_BM / 32; ++t)
+        if (t < nrt)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const int m = 32 * t + 8 * (i >> 2) + 4 * h + (i & 3);
+                if (m < mrows) g.y[(int64_t)s_p[m] * g.ldy + col] = acc[t][i];
+            }
+}
+
 // ------------------------------------------------------------------ launch
 template <int WT, int EPI>
 static int gb_launch(const GBArgs &a, hipStream_t st) {
@@ -537,6 +636,13 @@ static bool gb_side_ok(const GBArgs &g, const GBSide &s) {
 
 int launch_gb(const GBArgs &g, hipStream_t st) {
     if (g.max_tiles <= 0) return 0;
+    if (g.bm == GF_BM) {
+        if (g.a.type != 1 || g.glu || g.relu_sqr || g.sh_rows > 0 || !gb_side_ok(g, g)) return -6;
+        const int64_t nct = (g.ncols + 127) / 128;
+        if (nct > 0x7fffffff || g.max_tiles > 65535) return -6;
+        hipLaunchKernelGGL(k_gf, dim3((unsigned)nct, (unsigned)g.max_tiles), dim3(256), 0, st, g);
+        return hip_check_launch();
+    }
     if (g.bm != GB_BM_SMALL && g.bm != GB_BM_LARGE) return -6;
     if (!gb_side_ok(g, g)) return -6;
     if (g.sh_rows > 0 && (!gb_side_ok(g, g.sh) || g.sh.a.type != g.a.type || g.sh_rows > g.sh.xrows)) return -6;

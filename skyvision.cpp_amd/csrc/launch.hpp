@@ -345,6 +345,7 @@ struct GBArgs : GBSide {
     int sh_wgs, sh_tiles;      // (set by launch_gb)
 };
 constexpr int GB_BM_SMALL = 32, GB_BM_LARGE = 128;
+constexpr int GF_BM = 192;   // F16 tables, plain product, no shared expert: tiles of its own kernel (at most 65535)
 constexpr int64_t GB_MAX_X = 0xF0000000ll;          // bytes of xh (32-bit buffer offsets)
 constexpr int64_t GB_MAX_ROW_BYTES = 1ll << 25;
 int launch_gb(const GBArgs &g, hipStream_t st);

@@ -132,13 +132,51 @@ def test_mul_mat_id_bad_ids(t):
     wd = M.to_device(wq)
     ref = O.mul_mat_id(t, wq.reshape(E * N, -1), Kin, N, E, b, ids)
     ref[bad != ids] = 0.0
-    for kind in (2, 1):
+    for kind in (2, 1, 5):   # (5: F16 tables on the 192-row tiles)
         ctx.set_gemm_tiles(kind)
         M.check("mul_mat_id", ctx.mul_mat_id(M.tensor(wd, t, [Kin, N, E]), M.tensor(bd, M.TYPE_F32, [Kin, n_used, T]),
                                              M.tensor(idd, M.TYPE_I32, [n_used, T]), M.tensor(dst, M.TYPE_F32, [N, n_used, T])))
         got = dst.download(np.float32, (T, n_used, N))
         assert not got[bad != ids].any() and rel_l2(got, ref) <= TOL[t]
         assert ctx.take_errors()[0] == 2
+    ctx.close()
+
+
+@pytest.mark.parametrize("rows", [1, 31, 33, 96, 191, 192, 193, 400])
+@pytest.mark.parametrize("Kin,N", [(32, 128), (96, 130), (704, 33)])
+def test_mul_mat_id_f16_tiles(Kin, N, rows):
+    """F16 tables on the 192-row tiles of mul_mat_id (kind 5) against the oracle
+    and, bit for bit, the 32- and 128-row tiles: an odd block count, columns no
+    multiple of a work-group's, an expert of `rows` rows, one of one, one of none"""
+    _mul_mat_id_f16(Kin, N, 3, np.array([0] * rows + [2], np.int32).reshape(-1, 1), (2, 1, 5))
+
+
+@pytest.mark.parametrize("T", [256, 257, 900])
+def test_mul_mat_id_f16_rule(T):
+    """above 32 rows per expert the shape rule takes them (16 experts, 16 column groups)"""
+    ids = np.random.default_rng(T).permuted(np.tile(np.arange(16, dtype=np.int32), (T, 1)), axis=1)[:, :2].copy()
+    _mul_mat_id_f16(96, 2048, 16, ids, (2, 1, 5, 0))
+
+
+def _mul_mat_id_f16(Kin, N, E, ids, kinds):
+    rng = np.random.default_rng(Kin + N)
+    T, n_used = ids.shape
+    wq = _quant(M.TYPE_F16, (rng.standard_normal((E, N, Kin)) * 0.05).astype(np.float32))
+    b = rng.standard_normal((T, 1, Kin)).astype(np.float32)
+    ctx = M.Context(0)
+    ctx.reserve(T, max(Kin, 32), N, E, n_used)
+    ctx.set_gemm_threshold(1)
+    wd, bd, idd, dst = M.to_device(wq), M.to_device(b), M.to_device(ids), M.DeviceBuffer(4 * T * n_used * N)
+    ref = O.mul_mat_id(M.TYPE_F16, wq.reshape(E * N, -1), Kin, N, E, b, ids)
+    got = []
+    for kind in kinds:
+        ctx.set_gemm_tiles(kind)
+        M.check("mul_mat_id", ctx.mul_mat_id(M.tensor(wd, M.TYPE_F16, [Kin, N, E]), M.tensor(bd, M.TYPE_F32, [Kin, 1, T]),
+                                             M.tensor(idd, M.TYPE_I32, [n_used, T]), M.tensor(dst, M.TYPE_F32, [N, n_used, T])))
+        got.append(dst.download(np.float32, (T, n_used, N)))
+    assert rel_l2(got[0], ref) <= 1e-5   # (exact fp16 products, fp32 sums of Kin terms in another order)
+    for g in got[1:]:
+        assert np.array_equal(g.view(np.uint32), got[0].view(np.uint32))
     ctx.close()
 
 

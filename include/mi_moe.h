@@ -139,7 +139,9 @@ typedef struct {
  * otherwise do without; the results are bit-identical either way. */
 typedef struct {
     float   *logits;               /* [T][E]   router logits                      */
-    int32_t *sel;                  /* [T][K]   expert ids, descending logit        */
+    int32_t *sel;                  /* [T][K]   expert ids, descending logit (in
+                                               [0, E) and distinct also where a
+                                               token's logits are NaN)             */
     float   *weights;              /* [T][K]   softmax over the K selected logits  */
     int32_t *counts;               /* [E]      tokens routed to each expert        */
     int32_t *offsets;              /* [E+1]    exclusive prefix sum of counts      */
@@ -392,8 +394,9 @@ int mi_moe_ctx_stage_clock(mi_moe_ctx *ctx, const char *stage, double *ghz, int 
 /* Product path of a call: the grouped MFMA GEMM from min_tokens_for_gemm
  * tokens on, the grouped GEMV below.  0 (the default) picks by shape: for
  * k-quant layers the GEMM when 2 * T * K >= E (from half a dispatched row
- * per expert); for Q4_0 / Q5_0 / Q8_0 / F16 tables and mi_moe_mul_mat_id
- * when 4 * T * K > 5 * E (more than 1.25 rows per expert). */
+ * per expert); for Q4_0 / Q5_0 layers and mi_mul_mat_id when 4 * T * K > 5 * E
+ * (more than 1.25 rows per expert), for Q8_0 / F16 layers when 2 * T * K >
+ * 3 * E (more than 1.5). */
 int mi_moe_ctx_set_gemm_threshold(mi_moe_ctx *ctx, int64_t min_tokens_for_gemm);
 /* Row tiles of the grouped GEMMs.  Of Q4_K gate/up layers: 0 (the default) by
  * shape, 32-row tiles when the call dispatches at most 8 rows per expert on

@@ -632,8 +632,8 @@ B32Prep b32_x_prep(const mi_moe_ctx *c, const mi_moe_layer *L, int64_t T) {
 // routed FFN body of a layer with Q4_0 / Q5_0 / Q8_0 / F16 tables: the rows
 // converted to each product's ggml vec_dot_type (Q8_0 or fp16), fp32 slot
 // rows into the combine.  Below the GEMM threshold the grouped GEMV
-// (k_b32.hip), GLU rows in fp32; above it the grouped MFMA GEMM (k_gb.hip),
-// whose gate/up launch writes the down product's operand rows itself.
+// (k_b32.hip), above it the grouped MFMA GEMM (k_gb.hip); the gate/up launch of
+// either writes the down product's operand rows itself.
 // Arguments as run_experts; sh_here: the shared expert too (b32_shared_ok),
 // its rows' weights in sh_w (NULL: 1), added to the routed sum.
 int run_experts_b32(mi_moe_ctx *c, const mi_moe_layer *L, const float *x, int64_t T, const int32_t *ids_gu,

@@ -33,12 +33,13 @@
 // arithmetic): the weight stream, by the length of its runs - Q5_0 rows (K
 // 2688) in runs of 44, 88 and 176 bytes: 152, 121 and 105 us for 439 MB, as
 // contiguous memory 88 - and beside it the dequantization (Q5_0 104 us alone,
-// 142 with the stream); F16 streams at 5.4 TB/s.
+// 142 with the stream); F16 gate/up streams at 5.5 TB/s (1.02 GB in 186 us).
 // Against the form before (weights loaded by each lane for itself, dword by
-// dword, 192-row tiles): Q8_0 moondream3 T = 600 gate/up 268 -> 97 us, down
-// 127 -> 62 us, and the GLU rows' pass (13.7 us) is in the epilogue;
-// diffusiongemma F16 T = 256 257 -> 187 and 135 -> 104 us; nemotronomni Q5_0
-// T = 200 up 333 -> 134 us.
+// dword, 192-row tiles), kernel times under the profiler: Q8_0 moondream3 T =
+// 600 gate/up 268 -> 104 us, down 127 -> 66 us, and the GLU rows' pass (13.7
+// us) is in the epilogue; diffusiongemma F16 T = 256 257 -> 186 and 135 -> 107
+// us; nemotronomni Q5_0 T = 200 up 333 -> 134 us (165 with the shared expert
+// in it).
 #include "act.hpp"
 #include "b32.hpp"
 #include "common.hpp"

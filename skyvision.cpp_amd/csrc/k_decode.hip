@@ -659,8 +659,14 @@ __global__ void __launch_bounds__(DEC_THREADS) k_decode1(DecArgs g) {
             if (tpe >= 4) cnt += dpp_i<0x4E>(cnt);
             if (tpe >= 8) cnt += dpp_i<0x141>(cnt);
             if (e < E && j == 0 && cnt < K) {
-                s_sel[cnt] = e;
-                s_val[cnt] = ve;
+                // NaN logits (which count nothing above) rank behind the
+                // numbers, by id, as in topk_softmax_regs
+                if (__builtin_expect(ve != ve, 0))
+                    for (int i = 0; i < E; ++i) cnt += (int)(s_logit[i] == s_logit[i]) | (int)(i < e);
+                if (cnt < K) {
+                    s_sel[cnt] = e;
+                    s_val[cnt] = ve;
+                }
             }
         }
         dec_lds_barrier();

@@ -100,10 +100,11 @@ GATINGS = {"softmax": M.GATING_SOFTMAX_TOPK, "sigmoid": M.GATING_SIGMOID_BIAS, "
 
 @pytest.mark.parametrize("gating", list(GATINGS.values()), ids=list(GATINGS))
 @pytest.mark.parametrize("t,E,K,T,bad", [
+    (M.TYPE_Q4_K, 64, 8, 1, [0]), (M.TYPE_Q4_K, 20, 3, 1, [0]),                                         # one token
     (M.TYPE_Q4_K, 64, 8, 5, [1, 4]), (M.TYPE_Q4_K, 20, 3, 6, [0, 5]), (M.TYPE_Q4_K, 128, 4, 2, [1]),   # batched decode
     (M.TYPE_Q4_K, 64, 8, 70, [3, 64]), (M.TYPE_Q4_K, 200, 2, 24, [7]),                                  # the chain
     (M.TYPE_Q8_0, 64, 8, 4, [0]), (M.TYPE_Q8_0, 20, 3, 150, [0, 149])],
-    ids=["q4k-e64-t5", "q4k-e20-t6", "q4k-e128-t2", "q4k-e64-t70", "q4k-e200-t24", "q8-e64-t4", "q8-e20-t150"])
+    ids=["q4k-e64-t1", "q4k-e20-t1", "q4k-e64-t5", "q4k-e20-t6", "q4k-e128-t2", "q4k-e64-t70", "q4k-e200-t24", "q8-e64-t4", "q8-e20-t150"])
 def test_router_ids(t, E, K, T, bad, gating):
     D, I = 256, 256
     rng = np.random.default_rng(E + T)
@@ -142,6 +143,34 @@ def test_router_ids(t, E, K, T, bad, gating):
     if gating == M.GATING_SOFTMAX_TOPK:
         _check(run, x, bad)
     assert ctx.take_errors() == (0, 0)
+    ctx.close()
+
+
+@pytest.mark.parametrize("T", [1, 5, 70])
+@pytest.mark.parametrize("E,K,numbers", [(64, 8, 60), (64, 8, 8), (64, 8, 3), (20, 3, 2), (200, 4, 1)])
+def test_experts_without_a_logit(E, K, numbers, T):
+    """NaN logits of some experts rank behind the numbers, in the order of the ids: with at least K numbers left
+    ids, weights and outputs are those without the other experts; with fewer the token is NaN"""
+    D, I = 256, 256
+    rng = np.random.default_rng(E + numbers)
+    keep = []
+    L = _layer(rng, M.TYPE_Q4_K, D, I, E, K, keep)
+    bias = np.full(E, np.nan, np.float32)
+    bias[rng.permutation(E)[:numbers]] = 0.0
+    keep.append(M.to_device(bias))
+    L.router_b = keep[-1].addr
+    ctx = M.Context(0)
+    ctx.reserve(T, D, I, E, K)
+    out, sel, w, logits = _routed(ctx, L, rng.standard_normal((T, D)).astype(np.float32), D, E, K)
+    assert np.array_equal(np.isnan(logits), np.broadcast_to(np.isnan(bias), logits.shape))
+    key = np.where(np.isnan(logits), np.inf, -logits)
+    assert np.array_equal(sel, np.argsort(key, axis=1, kind="stable")[:, :K])
+    whole = numbers >= K
+    assert np.isfinite(w).all() == whole and np.isfinite(out).all() == whole
+    if whole:
+        assert np.allclose(w, O.softmax_selected(np.where(np.isnan(logits), -3e38, logits).astype(np.float32), sel), rtol=1e-6)
+    else:
+        assert np.isnan(w).all() and np.isnan(out).all()
     ctx.close()
 
 
